@@ -95,6 +95,61 @@ int mpc_fno_mix(const float *V, const float *Rr, const float *Ri, float *U, int 
 int mpc_fno_mix_bwd(const float *V, const float *dU, const float *Rr, const float *Ri, float *dV, float *dRr,
                     float *dRi, int nb, int w, int nxy, int mt, void *stream);
 
+/*
+ * One transverse point's work between two Fourier layers' transverse
+ * transforms, for all nb * npos points (npos = X Y).  Activations are
+ * [b][channel][pos][nt]; mode rows V6 and C1 are [b][channel][pos][n2].
+ *   V6 == NULL:  the lift, z = w v + bias from the 4 input channels v;
+ *   otherwise    z = V6 Gt + w v + bias  (w: width x width, row-major).
+ * out receives v' = GELU(z) if act else z, zs (layers only, may be NULL) z.
+ *   y == NULL:   C1 = v' Ft, the next layer's t-DFT;
+ *   otherwise    (no act) the head: y[b][0..2] = q2w GELU(q1w v' + q1) + q2 +
+ *                x[b][0..2], h hidden channels, x with batch stride x_bs.
+ * Gt (n2 x nt) and Ft (nt x n2) are given packed (mpc_fno_pack, which rounds
+ * them to BF16); V6 and v' are rounded to BF16 as operands of
+ * the t-DFTs, as mpc_gemm_bf16 does; the channel maps are FP32.  Supported
+ * where mpc_fno_column_fits says so (width 8, 16, 32 or 64, cin 4, nt <= 256,
+ * even n2 <= 64, h a
+ * power of two <= 64); otherwise MPC_EUNSUPP.
+ */
+typedef struct {
+    int nb, width, npos, nt, n2, act, h, pad_;
+    const float *v;
+    long v_bs;
+    const float *V6;
+    const float *w, *bias;
+    const void *Gt, *Ft;      /* packed, kinds 2 and 3 */
+    float *zs, *out, *C1;
+    const float *q1w, *q1, *q2w, *q2, *x;
+    long x_bs;
+    float *y;
+} mpc_fno_col;
+
+int mpc_fno_column(const mpc_fno_col *a, void *stream);
+int mpc_fno_column_fits(int w, int cin, int nt, int n2, int h);
+int mpc_sizeof_fno_col(void);
+
+/*
+ * Truncated complex DFT along one axis: the real-block product of G = [cos;
+ * sin] (2m x kk, given packed: mpc_fno_pack kind 0, or 1 for bwd) with every slice of in (nslice x kk rows of nq blocks
+ * [re(0..h) | im(0..h)]), operands rounded to BF16, and its recombination as
+ * mpc_fno_combine does it: out holds nslice x m rows.  bwd = 1: the transpose
+ * map (in: nslice x m rows, out: nslice x kk rows).  Supported where
+ * mpc_fno_dft_fits says so (the contracted length, kk or 2m, <= 128).
+ */
+int mpc_fno_dft(const void *G, const float *in, float *out, long nslice, int m, int kk, int nq, int h, int sign,
+                int bwd, void *stream);
+int mpc_fno_dft_fits(int m, int kk, int bwd);
+/*
+ * A constant matrix rounded to BF16 in the order these kernels read it: kind
+ * 0 / 1, G of mpc_fno_dft forward / bwd (m, kk as there); 2, Gt of
+ * mpc_fno_column (m = n2, kk = nt); 3, Ft (m = nt, kk = n2).  out is
+ * mpc_fno_pack_bytes(kind, m, kk) bytes of device memory (MPC_EUNSUPP where
+ * the kernels do not take the size).
+ */
+long mpc_fno_pack_bytes(int kind, int m, int kk);
+int  mpc_fno_pack(const float *G, void *out, int kind, int m, int kk, void *stream);
+
 /* z[b][c][p] += bias[c] (bias may be NULL), then out = GELU(z) if act else z */
 int mpc_fno_bias_act(float *z, const float *bias, float *out, long nb, int nc, long np, int act, void *stream);
 /* dz = dout * GELU'(z) if act else dout */

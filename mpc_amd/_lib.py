@@ -113,6 +113,13 @@ def lib() -> C.CDLL:
         "mpc_sizeof_gemm": (C.c_int, []),
         "mpc_gemm_bf16": (C.c_int, [vp, vp]),
         "mpc_fno_combine": (C.c_int, [vp, vp, C.c_long, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, vp]),
+        "mpc_sizeof_fno_col": (C.c_int, []),
+        "mpc_fno_column": (C.c_int, [vp, vp]),
+        "mpc_fno_column_fits": (C.c_int, [C.c_int] * 5),
+        "mpc_fno_dft": (C.c_int, [vp, vp, vp, C.c_long, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, vp]),
+        "mpc_fno_pack_bytes": (C.c_long, [C.c_int] * 3),
+        "mpc_fno_pack": (C.c_int, [vp, vp, C.c_int, C.c_int, C.c_int, vp]),
+        "mpc_fno_dft_fits": (C.c_int, [C.c_int] * 3),
         "mpc_fno_bias_act": (C.c_int, [vp, vp, vp, C.c_long, C.c_int, C.c_long, C.c_int, vp]),
         "mpc_fno_act_bwd": (C.c_int, [vp, vp, vp, C.c_long, C.c_int, vp]),
         "mpc_sizeof_pw": (C.c_int, []),

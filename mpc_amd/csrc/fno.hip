@@ -15,20 +15,11 @@
  * the loss and the Adam update.
  */
 #include "internal.h"
+#include "fno_device.h"
 #include "../../include/mpc_fno.h"
 #include <cmath>
 
 namespace {
-
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-/* FP32 -> BF16, round to nearest even (finite inputs) */
-__device__ __forceinline__ unsigned short to_bf16(float f) {
-    unsigned int u = __float_as_uint(f);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (unsigned short)(u >> 16);
-}
 
 constexpr int TM = 64, TN = 64, TK = 32;     /* workgroup tile */
 constexpr int LDK = TK + 4;                  /* LDS row length in bf16 (8-byte aligned rows) */
@@ -41,8 +32,8 @@ constexpr int LDK = TK + 4;                  /* LDS row length in bf16 (8-byte a
  * 2 x 2 MFMA 16 x 16 tiles.
  */
 __global__ void __launch_bounds__(256) k_gemm_bf16(mpc_gemm g) {
-    __shared__ __align__(16) unsigned short As[TM][LDK];
-    __shared__ __align__(16) unsigned short Bs[TN][LDK];   /* B^T: [n][k] */
+    __shared__ __align__(16) short As[TM][LDK];
+    __shared__ __align__(16) short Bs[TN][LDK];   /* B^T: [n][k] */
     const int nbat = g.nb1 * g.nb2;
     const int z = blockIdx.z;
     const int bat = z % nbat, split = z / nbat;
@@ -211,13 +202,6 @@ __global__ void k_combine(const float *__restrict__ in, float *__restrict__ out,
     }
 }
 
-__device__ __forceinline__ float gelu(float x) {
-    return 0.5f * x * (1.f + erff(x * 0.70710678118654752f));
-}
-__device__ __forceinline__ float gelu_d(float x) {
-    return 0.5f * (1.f + erff(x * 0.70710678118654752f)) + x * 0.39894228040143268f * expf(-0.5f * x * x);
-}
-
 /* z[b][c][p] += bias[c] (bias may be null); act: out = GELU(z) (or z) */
 __global__ void k_bias_act(float *__restrict__ z, const float *__restrict__ bias, float *__restrict__ out, long nb,
                            int nc, long np, int act) {
@@ -338,7 +322,6 @@ template <int CIN> static void launch_pointwise(const mpc_pw *a, dim3 grid, hipS
  * the lanes past the last point load the last point and skip their stores.
  * out may alias zin or zs: each element is read and written by one lane.
  */
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int PW_MF_WAVES = 4;
 
 template <int CIN, int OT>
@@ -434,42 +417,66 @@ template <int CIN> static void launch_pointwise_mf(const mpc_pw *a, hipStream_t 
  * Per-mode complex channel mixing of the spectral convolution, FP32.
  * V, U: [b][channel][kxy][2 mt] (re at kt, im at mt + kt); R = Rr + i Ri:
  * [i][o][kxy][mt].  Forward U[b][o] = sum_i V[b][i] R[i][o] (per mode).
- * One thread per (mode, o); the weights stream once (coalesced along the
- * mode), V is re-read per o from cache.
+ * A thread forms MIX_O output channels of one mode for all NB samples; the
+ * weights stream once (coalesced along the mode), V comes from cache once per
+ * MIX_O outputs.  Bound by the weights' HBM stream: eight input channels'
+ * loads are in flight per thread.
  */
-constexpr int MIX_BMAX = 8;
+constexpr int MIX_BMAX = 8, MIX_O = 2, MIX_I = 8;
+template <int NB>
 __global__ void __launch_bounds__(256) k_mix(const float *__restrict__ V, const float *__restrict__ Rr,
-                                             const float *__restrict__ Ri, float *__restrict__ U, int nb, int w,
-                                             int nxy, int mt) {
+                                             const float *__restrict__ Ri, float *__restrict__ U, int w, int nxy,
+                                             int mt) {
     const int nm = nxy * mt;
     const int m = blockIdx.x * 256 + threadIdx.x;
-    const int o = blockIdx.y;
+    const int o0 = blockIdx.y * MIX_O;
     if (m >= nm) return;
     const int kxy = m / mt, kt = m % mt;
     const long vm = (long)kxy * 2 * mt + kt;          /* re offset of the mode in a channel's block */
     const long cs = (long)nxy * 2 * mt;               /* channel stride in V, U */
-    float ur[MIX_BMAX], ui[MIX_BMAX];
+    float ur[MIX_O][NB], ui[MIX_O][NB];
 #pragma unroll
-    for (int b = 0; b < MIX_BMAX; ++b) ur[b] = ui[b] = 0.f;
-    for (int i = 0; i < w; ++i) {
-        const long ri = ((long)i * w + o) * nm + m;
-        const float rr = Rr[ri], rim = Ri[ri];
+    for (int j = 0; j < MIX_O; ++j)
 #pragma unroll
-        for (int b = 0; b < MIX_BMAX; ++b) {
-            if (b < nb) {
-                const float *v = V + ((long)b * w + i) * cs + vm;
-                const float vr = v[0], vi = v[mt];
-                ur[b] = fmaf(vr, rr, fmaf(-vi, rim, ur[b]));
-                ui[b] = fmaf(vr, rim, fmaf(vi, rr, ui[b]));
+        for (int b = 0; b < NB; ++b) ur[j][b] = ui[j][b] = 0.f;
+    for (int i0 = 0; i0 < w; i0 += MIX_I) {
+        float rr[MIX_I][MIX_O], ri[MIX_I][MIX_O], vr[MIX_I][NB], vi[MIX_I][NB];
+#pragma unroll
+        for (int i = 0; i < MIX_I; ++i) {
+            const int ii = min(i0 + i, w - 1);
+#pragma unroll
+            for (int j = 0; j < MIX_O; ++j) {
+                const long x = ((long)ii * w + min(o0 + j, w - 1)) * nm + m;
+                rr[i][j] = Rr[x];
+                ri[i][j] = Ri[x];
             }
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const float *v = V + ((long)b * w + ii) * cs + vm;
+                vr[i][b] = v[0];
+                vi[i][b] = v[mt];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < MIX_I; ++i) {
+            if (i0 + i >= w) break;
+#pragma unroll
+            for (int j = 0; j < MIX_O; ++j)
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    ur[j][b] = fmaf(vr[i][b], rr[i][j], fmaf(-vi[i][b], ri[i][j], ur[j][b]));
+                    ui[j][b] = fmaf(vr[i][b], ri[i][j], fmaf(vi[i][b], rr[i][j], ui[j][b]));
+                }
         }
     }
 #pragma unroll
-    for (int b = 0; b < MIX_BMAX; ++b) {
-        if (b < nb) {
-            float *u = U + ((long)b * w + o) * cs + vm;
-            u[0] = ur[b];
-            u[mt] = ui[b];
+    for (int j = 0; j < MIX_O; ++j) {
+        if (o0 + j >= w) break;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            float *u = U + ((long)b * w + o0 + j) * cs + vm;
+            u[0] = ur[j][b];
+            u[mt] = ui[j][b];
         }
     }
 }
@@ -703,8 +710,18 @@ extern "C" int mpc_fno_mix(const float *V, const float *Rr, const float *Ri, flo
                            int mt, void *stream) {
     if (!V || !Rr || !Ri || !U || nb <= 0 || nb > MIX_BMAX || w <= 0 || w > 65535 || nxy <= 0 || mt <= 0)
         return MPC_EINVAL;
-    const dim3 grid((unsigned)((nxy * mt + 255) / 256), (unsigned)w);
-    hipLaunchKernelGGL(k_mix, grid, dim3(256), 0, (hipStream_t)stream, V, Rr, Ri, U, nb, w, nxy, mt);
+    const dim3 grid((unsigned)((nxy * mt + 255) / 256), (unsigned)((w + MIX_O - 1) / MIX_O));
+    hipStream_t s = (hipStream_t)stream;
+    switch (nb) {
+    case 1: hipLaunchKernelGGL(k_mix<1>, grid, dim3(256), 0, s, V, Rr, Ri, U, w, nxy, mt); break;
+    case 2: hipLaunchKernelGGL(k_mix<2>, grid, dim3(256), 0, s, V, Rr, Ri, U, w, nxy, mt); break;
+    case 3: hipLaunchKernelGGL(k_mix<3>, grid, dim3(256), 0, s, V, Rr, Ri, U, w, nxy, mt); break;
+    case 4: hipLaunchKernelGGL(k_mix<4>, grid, dim3(256), 0, s, V, Rr, Ri, U, w, nxy, mt); break;
+    case 5: hipLaunchKernelGGL(k_mix<5>, grid, dim3(256), 0, s, V, Rr, Ri, U, w, nxy, mt); break;
+    case 6: hipLaunchKernelGGL(k_mix<6>, grid, dim3(256), 0, s, V, Rr, Ri, U, w, nxy, mt); break;
+    case 7: hipLaunchKernelGGL(k_mix<7>, grid, dim3(256), 0, s, V, Rr, Ri, U, w, nxy, mt); break;
+    default: hipLaunchKernelGGL(k_mix<8>, grid, dim3(256), 0, s, V, Rr, Ri, U, w, nxy, mt); break;
+    }
     return hipGetLastError() == hipSuccess ? 0 : MPC_EHIP;
 }
 

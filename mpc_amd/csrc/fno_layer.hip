@@ -1,0 +1,590 @@
+/*
+ * fno_layer.hip -- fused kernels of the pass surrogate's Fourier layers.
+ *
+ * k_column: everything between two layers' transverse transforms, one
+ * transverse point (x, y) at a time with all its channels and times: inverse
+ * t-DFT of the layer's mode coefficients, 1x1 channel map, bias, GELU, and
+ * the next layer's forward t-DFT (or, after the last layer, the projection
+ * head).  As separate kernels (k_gemm_bf16, k_pointwise_mf) these passes move
+ * the activations through HBM five times per layer; here they are read once
+ * and written once.
+ *
+ * k_dft / k_dft_t: a truncated complex DFT along y or x with the complex
+ * recombination in its epilogue, and its transpose.  As k_gemm_bf16 and
+ * k_combine the real-block products went through HBM between the two.
+ *
+ * The arithmetic is that of the separate kernels, in the same order: operands
+ * of the DFT products are rounded to BF16 as they are staged and products
+ * accumulate in FP32 along k in ascending order (the MFMA shapes
+ * v_mfma_f32_16x16x16_bf16, 16x16x32 and 32x32x16 give the same bits for the
+ * same order, checked on the device); the channel maps are FP32
+ * (v_mfma_f32_32x32x2f32: a chain of fused multiply-adds in ascending channel
+ * order, the same bits as the vector form).
+ */
+#include "internal.h"
+#include "fno_device.h"
+#include "../../include/mpc_fno.h"
+
+namespace {
+
+constexpr int CW = 8;                  /* waves per workgroup of k_column */
+constexpr int CT_MAX = 256;            /* t points a workgroup covers: CW tiles of 32 */
+constexpr int CN2_MAX = 64;            /* columns of the t-DFT (2 mt) */
+
+__device__ __forceinline__ f32x16 mfma_bf16(bf16x8 a, bf16x8 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+/* row of a 32 x 32 product that register r of a lane in half-wave h holds */
+__device__ __forceinline__ int drow(int r, int h) { return 8 * (r / 4) + 4 * h + r % 4; }
+
+/*
+ * k_column<W, CIN, KIND, ZS, CPI>: workgroups walk groups of CPI transverse
+ * points (b, pos), grid-stride.  Wave u of a workgroup holds t tile u % ntile
+ * (32 times) of point u / ntile of the group; a lane holds one time and, in
+ * each product register, one channel (drow).
+ *   KIND 0, lift:  z = Wm x + bias                        (no mode part)
+ *   KIND 1, layer: z = V6 Gt + Wm v + bias; v' = GELU(z) if act; ZS (training):
+ *           z is stored too and the GELU is the training path's
+ *   KIND 2, last:  as KIND 1, then y = Q2 GELU(Q1 v' + q1) + q2 + x[:, :2]
+ * Kinds 0 and 1 then form C1 = v' Ft, from v' rounded to BF16 in LDS.
+ * LDS at W = 32, T = 256: Ft 33 KB, v' 17 KB, V6 5 KB, Wm 4 KB: two workgroups
+ * (four waves per SIMD) fit on a CU, so one's loads and stores run under the
+ * other's products and GELUs.
+ *
+ * The next group's mode rows and channels are loaded while this one is worked
+ * on.  Loads and stores share one in-order counter, so a wait for those loads
+ * must not also wait for the stores behind them: the loop is straight-line
+ * (in a branch the compiler has to assume the path without the stores).
+ * Times past T, waves without a tile, rows past W and columns past n2
+ * therefore work on the last valid one again and store the same value there.
+ */
+template <int W, int CIN, int KIND> struct ColCfg {
+    static constexpr int MT = W <= 32 ? 1 : W / 32;            /* 32-row channel tiles */
+    static constexpr int NR = W >= 32 ? 16 : W / 2;            /* product registers in use per tile */
+    static constexpr int KS = (CIN + 1) / 2;                   /* FP32 product steps of the channel map */
+    static constexpr int WP = CIN + 1;                         /* LDS pitch of the weight rows */
+    static constexpr int AP = CN2_MAX + 8;                     /* pitch of the staged V6 rows */
+    static constexpr int M16 = (W + 15) / 16;                  /* 16-row tiles of the forward t-DFT */
+};
+
+template <int W, int CIN, int KIND, bool ZS, int CPI>
+__global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col a) {
+    using C = ColCfg<W, CIN, KIND>;
+    constexpr int MT = C::MT, NR = C::NR, KS = C::KS, WP = C::WP, AP = C::AP, M16 = C::M16;
+    const int T = a.nt, n2 = a.n2, npos = a.npos;
+    const int ntile = (T + 31) / 32, tpad = 32 * ntile;
+    const int tp = tpad + 8;                                   /* pitch of the v' and Ft rows (bf16) */
+    const int n16 = (n2 + 15) / 16;
+    extern __shared__ __align__(16) unsigned char smem[];
+    /* bias | Wm | q1 and its weights (KIND 2) | V6 rows | v' rows | Ft rows */
+    float *Bl = reinterpret_cast<float *>(smem);
+    float *Wl = Bl + MT * 32;
+    float *Ql = Wl + MT * 32 * WP;
+    const int ht = KIND == 2 ? (a.h + 31) / 32 : 0;
+    short *A6 = reinterpret_cast<short *>(smem + ((MT * 32 * (WP + 1) + ht * 32 * (W + 4)) * 4 + 15) / 16 * 16);
+    short *Vl = A6 + (KIND ? CPI * MT * 32 * AP : 0);
+    short *Fl = Vl + CPI * M16 * 16 * tp;
+
+    const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, half = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int unit = min(wave, CPI * ntile - 1);
+    const int csub = unit / ntile, tile = unit % ntile;
+    const int t = 32 * tile + col;
+
+    for (int i = tid; i < MT * 32; i += 64 * CW) Bl[i] = i < W ? a.bias[i] : 0.f;
+    for (int i = tid; i < MT * 32 * CIN; i += 64 * CW) {
+        const int o = i / CIN, k = i % CIN;
+        Wl[o * WP + k] = o < W ? a.w[o * CIN + k] : 0.f;
+    }
+    /* q1 | the two rows of Q2 | Q1 */
+    if constexpr (KIND == 2) {
+        for (int i = tid; i < ht * 32 * W; i += 64 * CW) {
+            const int o = i / W, k = i % W;
+            Ql[ht * 96 + o * (W + 1) + k] = o < a.h ? a.q1w[o * W + k] : 0.f;
+        }
+        for (int o = tid; o < ht * 32; o += 64 * CW) {
+            Ql[o] = o < a.h ? a.q1[o] : 0.f;
+            Ql[ht * 32 + o] = o < a.h ? a.q2w[o] : 0.f;
+            Ql[ht * 64 + o] = o < a.h ? a.q2w[a.h + o] : 0.f;
+        }
+    }
+    if constexpr (KIND != 0)
+        for (int i = tid; i < CPI * MT * 32 * AP; i += 64 * CW) A6[i] = 0;
+    if constexpr (KIND != 2) {
+        const int rq = tpad / 8;                               /* 16-byte pieces per row */
+        for (int i = tid; i < n16 * 16 * rq; i += 64 * CW)
+            *reinterpret_cast<bf16x8 *>(Fl + i / rq * tp + i % rq * 8) = reinterpret_cast<const bf16x8 *>(a.Ft)[i];
+    }
+    /* the wave's columns of Gt */
+    bf16x8 gB[KIND ? 4 : 1];
+    if constexpr (KIND != 0) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) gB[s] = reinterpret_cast<const bf16x8 *>(a.Gt)[(tile * 4 + s) * 64 + lane];
+    }
+
+    const int stride = gridDim.x * CPI;
+    const unsigned cs = (unsigned)npos * (unsigned)T;          /* channel stride of the activations */
+    /* byte offsets of this lane's time from a sample's (b, pos), in channel row
+     * half and channel row 4 half; a channel is c4 bytes */
+    const unsigned to = 4u * (unsigned)min(t, T - 1);
+    const unsigned xo = 4u * half * cs + to, lo = 16u * half * cs + to, c4 = 4u * cs;
+    auto advance = [&](int &b, int &pos, int by) {
+        pos += by;
+        while (pos >= npos) { pos -= npos; ++b; }
+    };
+    /* point i of the group at (b0, pos0), or the last point there is */
+    auto point = [&](int b0, int pos0, int i, int &b, int &pos) {
+        b = b0;
+        pos = pos0;
+        advance(b, pos, i);
+        if (b >= a.nb) { b = a.nb - 1; pos = npos - 1; }
+    };
+    /* V6 of a group: CPI x W rows of n2 floats (n2 even); 32 threads a row, two floats each */
+    constexpr int RPP = 64 * CW / 32, NV = (CPI * W + RPP - 1) / RPP;
+    float2 pre[KIND ? NV : 1];
+    const int kp = min(tid & 31, n2 / 2 - 1), row0 = tid >> 5;
+    const unsigned row4 = 4u * (unsigned)npos * (unsigned)n2;  /* bytes of a channel's mode rows */
+    auto load_v6 = [&](int b0, int pos0) {
+        if constexpr (KIND != 0) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+                const int r = min(row0 + RPP * i, CPI * W - 1);
+                int b, pos;
+                point(b0, pos0, CPI > 1 ? __builtin_amdgcn_readfirstlane(r / W) : 0, b, pos);   /* a wave's two rows are of one point */
+                pre[i] = buf_ld2(buf_of(a.V6 + (long)b * W * npos * n2), (unsigned)(r % W) * row4 + 8u * kp, 4u * pos * n2);
+            }
+        }
+    };
+    float xv[KS], xn[KS];                                      /* this wave's channels of its time; the next group's */
+    auto load_x = [&](int b0, int pos0) {
+        int b, pos;
+        point(b0, pos0, csub, b, pos);
+        const rsrc_t xb = buf_of(a.v + b * a.v_bs);
+#pragma unroll
+        for (int s = 0; s < KS; ++s) xn[s] = buf_ld(xb, xo, 4u * pos * T + 2u * s * c4);
+    };
+    int b0 = 0, pos0 = 0;                                      /* the group's first point */
+    advance(b0, pos0, blockIdx.x * CPI);
+    __syncthreads();                                           /* the zeroed rows come before the staged ones */
+    load_v6(b0, pos0);
+    load_x(b0, pos0);
+    /* the loads of the next group are waited for here, at the end of a
+     * group's work, where the stores issued after them are known and need not
+     * be waited for: at the top of the loop the wait would have to suit the
+     * first round too, which has none */
+    auto arrive = [&] {
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            asm volatile("" : "+v"(xn[s]));
+            xv[s] = xn[s];
+        }
+        if constexpr (KIND != 0) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(pre[i].x), "+v"(pre[i].y));
+        }
+    };
+    arrive();
+    while (b0 < a.nb) {
+        if constexpr (KIND != 0) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+                const int r = min(row0 + RPP * i, CPI * W - 1);
+                *reinterpret_cast<int *>(&A6[(r / W * MT * 32 + r % W) * AP + 2 * kp]) = bf16_pair(pre[i].x, pre[i].y);
+            }
+        }
+        __syncthreads();
+        int bn = b0, pn = pos0;
+        advance(bn, pn, stride);
+        load_v6(bn, pn);
+        load_x(bn, pn);
+        int b, pos;
+        point(b0, pos0, csub, b, pos);
+        const long ob = (long)b * W * cs;
+        const unsigned po = 4u * pos * T;
+        float zr[KIND == 2 ? MT : 1][16];
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            f32x16 sp = {}, acc = {};
+            if constexpr (KIND != 0) {
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    sp = mfma_bf16(*reinterpret_cast<const bf16x8 *>(&A6[((csub * MT + m) * 32 + col) * AP + 16 * s + 8 * half]),
+                                   gB[s], sp);
+            }
+#pragma unroll
+            for (int s = 0; s < KS; ++s)
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(Wl[(32 * m + col) * WP + 2 * s + half], xv[s], acc, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                if constexpr (KIND != 0) acc[r] += sp[r];
+                acc[r] += Bl[32 * m + 4 * half + 8 * (r / 4) + r % 4];
+            }
+            /* rows of the lower half-wave: 32 m + 8 (r / 4) + r % 4 */
+            auto store = [&](float *base) {
+                const rsrc_t rs = buf_of(base + ob);
+#pragma unroll
+                for (int r = 0; r < NR; ++r) buf_st(rs, lo, po + (32u * m + 8 * (r / 4) + r % 4) * c4, acc[r]);
+            };
+            if constexpr (ZS) store(a.zs);
+            if constexpr (KIND == 2) {
+#pragma unroll
+                for (int r = 0; r < NR; ++r) zr[m][r] = acc[r];
+            } else {
+                if (a.act) {
+#pragma unroll
+                    for (int r = 0; r < NR; ++r) acc[r] = ZS ? gelu(acc[r]) : gelu_fast(acc[r]);
+                }
+                store(a.out);
+                short *vl = Vl + (csub * M16 * 16 + 32 * m + 4 * half) * tp + t;
+#pragma unroll
+                for (int r = 0; r < NR; ++r) vl[(8 * (r / 4) + r % 4) * tp] = to_bf16(acc[r]);
+            }
+        }
+        if constexpr (KIND == 2) {
+            /* the channels of a time lie in the registers of two lanes; as the
+             * operand of the next channel map, step s takes channels 2s (lower
+             * half-wave) and 2s + 1 (upper): pairs of registers swap halves */
+            float xb2[MT * NR];
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int r = 0; r < NR; r += 2) {
+                    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(zr[m][r]), __float_as_uint(zr[m][r + 1]), false, false);
+                    const int s0 = 16 * m + 4 * (r / 4) + (r % 4) / 2;
+                    xb2[s0] = __uint_as_float(p[0]);
+                    xb2[s0 + 2] = __uint_as_float(p[1]);
+                }
+            float y0 = 0.f, y1 = 0.f;
+            for (int q = 0; q < ht; ++q) {
+                f32x16 acc = {};
+#pragma unroll
+                for (int s = 0; s < W / 2; ++s)
+                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(Ql[ht * 96 + (32 * q + col) * (W + 1) + 2 * s + half], xb2[s], acc, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int o = 32 * q + drow(r, half);
+                    const float hv = gelu_fast(acc[r] + Ql[o]);
+                    y0 = fmaf(Ql[ht * 32 + o], hv, y0);
+                    y1 = fmaf(Ql[ht * 64 + o], hv, y1);
+                    /* the rows' LDS operands load where they are used, not all ahead */
+                    if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            /* each half-wave summed its rows of both outputs: the lower one
+             * finishes output 0, the upper one output 1 */
+            const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(y0), __float_as_uint(y1), false, false);
+            const float ys = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+            const float x0 = buf_ld(buf_of(a.x + b * a.x_bs), xo, po);
+            buf_st(buf_of(a.y + b * 2L * cs), xo, po, ys + x0 + a.q2[half]);
+        }
+        __syncthreads();
+        if constexpr (KIND != 2) {
+            constexpr int RND = (CPI * M16 * (CN2_MAX / 16) + CW - 1) / CW;
+            const int nt16 = CPI * M16 * n16;
+#pragma unroll
+            for (int r = 0; r < RND; ++r) {
+                const int i = min(wave + r * CW, nt16 - 1);
+                const int n = i % n16, cm = i / n16, cc = cm / M16, m = cm % M16;
+                int b2, p2;
+                point(b0, pos0, cc, b2, p2);
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                const short *ap = Vl + ((cc * M16 + m) * 16 + (lane & (W < 16 ? 7 : 15))) * tp + 8 * (lane >> 4);
+                const short *bp = Fl + (n * 16 + (lane & 15)) * tp + 8 * (lane >> 4);
+                for (int k = 0; k < tpad; k += 32)
+                    acc = mfma_bf16(*reinterpret_cast<const bf16x8 *>(ap + k), *reinterpret_cast<const bf16x8 *>(bp + k), acc);
+                const int nn = min(n * 16 + (lane & 15), n2 - 1);
+                const unsigned o = (unsigned)(4 * (lane >> 4) % W) * row4 + 4u * nn;
+                const rsrc_t cp = buf_of(a.C1 + (long)b2 * W * npos * n2);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) buf_st(cp, o, 4u * p2 * n2 + (16u * m + e) * row4, acc[e]);
+            }
+        }
+        arrive();
+        b0 = bn;
+        pos0 = pn;
+    }
+}
+
+template <int W, int CIN, int KIND, bool ZS, int CPI> int column_go(const mpc_fno_col *a, hipStream_t s) {
+    using C = ColCfg<W, CIN, KIND>;
+    const int tp = (a->nt + 31) / 32 * 32 + 8, ht = KIND == 2 ? (a->h + 31) / 32 : 0, n16 = (a->n2 + 15) / 16;
+    size_t lds = ((size_t)(C::MT * 32 * (C::WP + 1) + ht * 32 * (W + 4)) * 4 + 15) / 16 * 16;
+    if (KIND) lds += (size_t)CPI * C::MT * 32 * C::AP * 2;
+    if (KIND != 2) lds += (size_t)(CPI * C::M16 * 16 + n16 * 16) * tp * 2;
+    int dev = 0, ncu = 0, per = 0;
+    const void *k = (const void *)k_column<W, CIN, KIND, ZS, CPI>;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, 64 * CW, lds) != hipSuccess || per < 1)
+        return MPC_EHIP;
+    const long ngrp = ((long)a->nb * a->npos + CPI - 1) / CPI;
+    const unsigned grid = (unsigned)std::min(ngrp, (long)ncu * per);
+    hipLaunchKernelGGL((k_column<W, CIN, KIND, ZS, CPI>), dim3(grid), dim3(64 * CW), lds, s, *a);
+    return hipGetLastError() == hipSuccess ? 0 : MPC_EHIP;
+}
+/* short lines (at most CW/2 t tiles): two points at a time, so that no wave idles */
+template <int W, int CIN, int KIND, bool ZS> int column_k(const mpc_fno_col *a, hipStream_t s) {
+    return (a->nt + 31) / 32 <= CW / 2 ? column_go<W, CIN, KIND, ZS, 2>(a, s) : column_go<W, CIN, KIND, ZS, 1>(a, s);
+}
+template <int W> int column_w(const mpc_fno_col *a, hipStream_t s) {
+    if (!a->V6) return column_k<W, 4, 0, false>(a, s);
+    if (a->y) return column_k<W, W, 2, false>(a, s);
+    return a->zs ? column_k<W, W, 1, true>(a, s) : column_k<W, W, 1, false>(a, s);
+}
+
+/* ---------------------------------------------------------------------- */
+/* truncated DFT along y or x                                              */
+/* ---------------------------------------------------------------------- */
+/*
+ * out[s][row][q][re(0..h) | im(0..h)], row < m, from in[s][k][q][re | im],
+ * k < kk, and G = [cos (m x kk); sin (m x kk)]:
+ *   out = (C in)_r - sg (S in)_i,  (C in)_i + sg (S in)_r.
+ * A wave forms 16 rows x 32 columns of a block's re and im parts: its 32 x 32
+ * product tile holds the 16 cos rows in registers 0-7 and the same 16 sin rows
+ * in registers 8-15, so the recombination stays within a lane.  Inputs go
+ * from memory to registers (an element is an operand of at most m / 16 waves)
+ * and a wave walks slices with its rows of G in registers, so there is no
+ * LDS and no barrier.  kk <= 16 KS.
+ */
+/* FULL: kk = 16 KS */
+template <int KS, bool FULL>
+__global__ void __launch_bounds__(256) k_dft(const bf16x8 *__restrict__ G, const float *__restrict__ in,
+                                             float *__restrict__ out, long nunit, int m, int kk, int nq, int h, float sg) {
+    const int lane = threadIdx.x & 63, col = lane & 31, half = lane >> 5;
+    const int m0 = blockIdx.y * 16;
+    bf16x8 ga[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) ga[s] = G[(blockIdx.y * KS + s) * 64 + lane];
+    const int nh = (h + 31) / 32;
+    const long rowl = (long)nq * 2 * h;                        /* floats per row of a slice */
+    /* unit: (slice, block q, column tile) */
+    for (long u = blockIdx.x * 4L + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); u < nunit; u += gridDim.x * 4L) {
+        const int hc = (int)(u % nh);
+        const long sq = u / nh;
+        const int q = (int)(sq % nq);
+        const long sl = sq / nq;
+        const int c = hc * 32 + col;
+        const bool cin = c < h;
+        const rsrc_t ib = buf_of(in + sl * kk * rowl + q * 2 * h);
+        f32x16 re = {}, im = {};
+        float vr[KS][8], vi[KS][8];
+        /* rows past kk meet zero columns of G: the last row stands in for them */
+        const unsigned co = 4u * (unsigned)(cin ? c : h - 1), row4 = 4u * (unsigned)rowl;
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const unsigned o = FULL ? (unsigned)(8 * half) * row4 + co
+                                        : (unsigned)min(16 * s + 8 * half + j, kk - 1) * row4 + co;
+                const unsigned u0 = FULL ? (16 * s + j) * row4 : 0;
+                vr[s][j] = buf_ld(ib, o, u0);
+                vi[s][j] = buf_ld(ib, o, u0 + 4 * h);
+            }
+        if constexpr (KS <= 4) __builtin_amdgcn_sched_barrier(0);    /* all loads go out before the first wait */
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            re = mfma_bf16(ga[s], bf16_octet(vr[s]), re);
+            im = mfma_bf16(ga[s], bf16_octet(vi[s]), im);
+        }
+        const rsrc_t ob = buf_of(out + (sl * m + m0) * rowl + q * 2 * h);
+        const unsigned oo = (unsigned)(4 * half) * row4 + co;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const int row = 8 * (r / 4) + r % 4;
+            if (cin && m0 + row + 4 * half < m) {
+                buf_st(ob, oo, row * row4, re[r] - sg * im[r + 8]);
+                buf_st(ob, oo, row * row4 + 4 * h, im[r] + sg * re[r + 8]);
+            }
+        }
+    }
+}
+
+/*
+ * The transpose: out[s][k][q][re | im] = sum over the 2m real rows of G of
+ * G[row][k] dP[row], dP the transposed recombination of in[s][row][q][re | im]
+ * (row < m: (dVr, dVi); row >= m: (sg dVi, -sg dVr)).  A wave forms 32 k x 32
+ * columns of re and im.  2 m <= 16 KS.
+ */
+template <int KS>
+__global__ void __launch_bounds__(256) k_dft_t(const bf16x8 *__restrict__ G, const float *__restrict__ in,
+                                               float *__restrict__ out, long nunit, int m, int kk, int nq, int h, float sg) {
+    const int lane = threadIdx.x & 63, col = lane & 31, half = lane >> 5;
+    const int k0 = blockIdx.y * 32;
+    const int m2 = 2 * m;
+    bf16x8 ga[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) ga[s] = G[(blockIdx.y * KS + s) * 64 + lane];
+    const int nh = (h + 31) / 32;
+    const long rowl = (long)nq * 2 * h;
+    for (long u = blockIdx.x * 4L + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); u < nunit; u += gridDim.x * 4L) {
+        const int hc = (int)(u % nh);
+        const long sq = u / nh;
+        const int q = (int)(sq % nq);
+        const long sl = sq / nq;
+        const int c = hc * 32 + col;
+        const bool cin = c < h;
+        const rsrc_t ib = buf_of(in + sl * m * rowl + q * 2 * h);
+        f32x16 re = {}, im = {};
+        const unsigned co = 4u * (unsigned)(cin ? c : h - 1), row4 = 4u * (unsigned)rowl;
+        float vr[KS][8], vi[KS][8];
+        /* rows past 2m meet zero columns: the last row stands in for them */
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int r = min(16 * s + 8 * half + j, m2 - 1);
+                const bool sine = r >= m;
+                const unsigned o = (unsigned)(sine ? r - m : r) * row4 + co;
+                const float x = buf_ld(ib, o, 0), y = buf_ld(ib, o, 4 * h);
+                vr[s][j] = sine ? sg * y : x;
+                vi[s][j] = sine ? -sg * x : y;
+            }
+        if constexpr (KS <= 4) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            re = mfma_bf16(ga[s], bf16_octet(vr[s]), re);
+            im = mfma_bf16(ga[s], bf16_octet(vi[s]), im);
+        }
+        const rsrc_t ob = buf_of(out + (sl * kk + k0) * rowl + q * 2 * h);
+        const unsigned oo = (unsigned)(4 * half) * row4 + co;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int k = 8 * (r / 4) + r % 4;
+            if (cin && k0 + k + 4 * half < kk) {
+                buf_st(ob, oo, k * row4, re[r]);
+                buf_st(ob, oo, k * row4 + 4 * h, im[r]);
+            }
+        }
+    }
+}
+
+/* K steps a k_dft instantiation holds for a contraction over n */
+int dft_steps(int n) { return n <= 16 ? 1 : n <= 32 ? 2 : n <= 64 ? 4 : 8; }
+int dft_tiles(int m, int kk, bool tr) { return tr ? (kk + 31) / 32 : (m + 15) / 16; }
+
+/*
+ * The constant operands in the order the products read them, 8 BF16 per lane
+ * and step, so a wave's rows load as 1 KB pieces.  Read as rows of the FP32
+ * matrix, every lane of a load touches a cache line of its own, and those
+ * accesses were most of a k_dft launch (28 us of which 20 at 64 x 64 x 256,
+ * width 32).
+ * kind 0: rows of G = [cos; sin] for k_dft (16 cos rows, the same 16 sin rows
+ * per tile); 1: columns of G for k_dft_t; 2: Gt (n2 x nt) for k_column, 4
+ * steps of 16 per 32-point t tile; 3: Ft (nt x n2), transposed, for k_column's
+ * LDS.  Contracted indices past the end are zero; times past nt (kind 2) and
+ * columns past n2 (3) repeat the last one.
+ */
+__global__ void k_pack(const float *__restrict__ G, short *__restrict__ out, long n, int kind, int m, int kk, int steps) {
+    for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L) {
+        const int j = (int)(i % 8), lane = (int)(i / 8 % 64), col = lane & 31, half = lane >> 5;
+        const int step = (int)(i / 512 % steps), tile = (int)(i / 512 / steps);
+        const int c = 16 * step + 8 * half + j;                /* contracted index */
+        float v = 0.f;
+        if (kind == 0) {
+            const int row = tile * 16 + (col & 15);
+            if (row < m && c < kk) v = G[(long)(col < 16 ? row : m + row) * kk + c];
+        } else if (kind == 1) {
+            const int k = tile * 32 + col;
+            if (c < 2 * m && k < kk) v = G[(long)c * kk + k];
+        } else if (kind == 2) {                                /* m = n2, kk = nt */
+            const int t = min(tile * 32 + col, kk - 1);
+            if (c < m) v = G[(long)c * kk + t];
+        } else {                                               /* m = nt, kk = n2: rows of tpad */
+            const int tpad = (m + 31) / 32 * 32;
+            const int t = (int)(i % tpad), nn = min((int)(i / tpad), kk - 1);
+            if (t < m) v = G[(long)t * kk + nn];
+        }
+        out[i] = to_bf16(v);
+    }
+}
+long pack_elems(int kind, int m, int kk, int *steps) {
+    *steps = 4;
+    switch (kind) {
+    case 0: *steps = dft_steps(kk); return (long)dft_tiles(m, kk, false) * *steps * 512;
+    case 1: *steps = dft_steps(2 * m); return (long)dft_tiles(m, kk, true) * *steps * 512;
+    case 2: return (long)((kk + 31) / 32) * 4 * 512;
+    default: return (long)((kk + 15) / 16 * 16) * ((m + 31) / 32 * 32);
+    }
+}
+
+template <int KS>
+void dft_go(bool tr, const void *G, const float *in, float *out, long nunit, int m, int kk, int nq, int h, float sg,
+            hipStream_t s) {
+    const int tiles = dft_tiles(m, kk, tr);
+    /* a wave keeps its rows of G for several units once the chip is full */
+    const long blocks = std::max(1L, std::min((nunit + 3) / 4, 4096L / tiles));
+    const dim3 grid((unsigned)blocks, (unsigned)tiles);
+    const bf16x8 *g = (const bf16x8 *)G;
+    if (tr) hipLaunchKernelGGL((k_dft_t<KS>), grid, dim3(256), 0, s, g, in, out, nunit, m, kk, nq, h, sg);
+    else if (kk == 16 * KS)
+        hipLaunchKernelGGL((k_dft<KS, true>), grid, dim3(256), 0, s, g, in, out, nunit, m, kk, nq, h, sg);
+    else hipLaunchKernelGGL((k_dft<KS, false>), grid, dim3(256), 0, s, g, in, out, nunit, m, kk, nq, h, sg);
+}
+
+} // namespace
+
+extern "C" int mpc_sizeof_fno_col(void) { return (int)sizeof(mpc_fno_col); }
+
+extern "C" int mpc_fno_column_fits(int w, int cin, int nt, int n2, int h) {
+    return (w == 8 || w == 16 || w == 32 || w == 64) && cin == 4 && nt >= 1 && nt <= CT_MAX && n2 >= 2 && n2 % 2 == 0 &&
+           n2 <= CN2_MAX && h >= 1 && h <= 64 && (h & (h - 1)) == 0;
+}
+
+extern "C" int mpc_fno_column(const mpc_fno_col *a, void *stream) {
+    if (!a || a->nb <= 0 || a->npos <= 0 || !a->v || !a->w || !a->bias) return MPC_EINVAL;
+    if (!mpc_fno_column_fits(a->width, 4, a->nt, a->n2, a->y ? a->h : 1)) return MPC_EUNSUPP;
+    /* byte offsets within a sample's activations and mode rows are 32-bit */
+    if ((long)a->width * a->npos * std::max(a->nt, a->n2) > (1L << 29) || (long)a->nb * a->npos > (1L << 30))
+        return MPC_EUNSUPP;
+    if (a->zs && (!a->V6 || a->y)) return MPC_EINVAL;
+    if (a->V6 && !a->Gt) return MPC_EINVAL;
+    if (a->y ? (!a->q1w || !a->q1 || !a->q2w || !a->q2 || !a->x || !a->V6) : (!a->Ft || !a->C1 || !a->out)) return MPC_EINVAL;
+    hipStream_t s = (hipStream_t)stream;
+    switch (a->width) {
+    case 8:  return column_w<8>(a, s);
+    case 16: return column_w<16>(a, s);
+    case 32: return column_w<32>(a, s);
+    default: return column_w<64>(a, s);
+    }
+}
+
+extern "C" int mpc_fno_dft_fits(int m, int kk, int bwd) {
+    return m >= 1 && kk >= 1 && (bwd ? 2 * m : kk) <= 128 && m <= (1 << 20) && kk <= (1 << 20);
+}
+
+extern "C" long mpc_fno_pack_bytes(int kind, int m, int kk) {
+    if (kind < 0 || kind > 3 || m <= 0 || kk <= 0 || (kind < 2 && !mpc_fno_dft_fits(m, kk, kind)) ||
+        (kind == 2 && (m > CN2_MAX || kk > CT_MAX)) || (kind == 3 && (kk > CN2_MAX || m > CT_MAX)))
+        return MPC_EUNSUPP;
+    int steps;
+    return 2 * pack_elems(kind, m, kk, &steps);
+}
+
+extern "C" int mpc_fno_pack(const float *G, void *out, int kind, int m, int kk, void *stream) {
+    if (!G || !out || mpc_fno_pack_bytes(kind, m, kk) <= 0) return MPC_EINVAL;
+    int steps;
+    const long n = pack_elems(kind, m, kk, &steps);
+    hipLaunchKernelGGL(k_pack, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, G, (short *)out, n,
+                       kind, m, kk, steps);
+    return hipGetLastError() == hipSuccess ? 0 : MPC_EHIP;
+}
+
+extern "C" int mpc_fno_dft(const void *G, const float *in, float *out, long nslice, int m, int kk, int nq, int h,
+                           int sign, int bwd, void *stream) {
+    if (!G || !in || !out || in == out || nslice <= 0 || nq <= 0 || h <= 0 || (sign != 1 && sign != -1)) return MPC_EINVAL;
+    /* byte offsets within a slice are 32-bit */
+    if (!mpc_fno_dft_fits(m, kk, bwd) || (long)std::max(m, kk) * nq * 2 * h > (1L << 29)) return MPC_EUNSUPP;
+    hipStream_t s = (hipStream_t)stream;
+    const long nunit = nslice * nq * ((h + 31) / 32);
+    const float sg = (float)sign;
+    switch (dft_steps(bwd ? 2 * m : kk)) {
+    case 1:  dft_go<1>(bwd != 0, G, in, out, nunit, m, kk, nq, h, sg, s); break;
+    case 2:  dft_go<2>(bwd != 0, G, in, out, nunit, m, kk, nq, h, sg, s); break;
+    case 4:  dft_go<4>(bwd != 0, G, in, out, nunit, m, kk, nq, h, sg, s); break;
+    default: dft_go<8>(bwd != 0, G, in, out, nunit, m, kk, nq, h, sg, s); break;
+    }
+    return hipGetLastError() == hipSuccess ? 0 : MPC_EHIP;
+}

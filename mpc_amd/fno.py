@@ -47,6 +47,14 @@ class MpcPw(C.Structure):
                 ("zs", C.c_void_p), ("out", C.c_void_p), ("act", C.c_int)]
 
 
+class MpcFnoCol(C.Structure):
+    _fields_ = [("nb", C.c_int), ("width", C.c_int), ("npos", C.c_int), ("nt", C.c_int), ("n2", C.c_int),
+                ("act", C.c_int), ("h", C.c_int), ("pad_", C.c_int), ("v", C.c_void_p), ("v_bs", C.c_long),
+                ("V6", C.c_void_p), ("w", C.c_void_p), ("bias", C.c_void_p), ("Gt", C.c_void_p), ("Ft", C.c_void_p),
+                ("zs", C.c_void_p), ("out", C.c_void_p), ("C1", C.c_void_p), ("q1w", C.c_void_p), ("q1", C.c_void_p),
+                ("q2w", C.c_void_p), ("q2", C.c_void_p), ("x", C.c_void_p), ("x_bs", C.c_long), ("y", C.c_void_p)]
+
+
 MIX_BMAX = 8          # samples per mode-mixing launch
 
 
@@ -123,6 +131,8 @@ class Ops:
             raise RuntimeError("mpc_gemm layout mismatch between library and binding")
         if lib().mpc_sizeof_pw() != C.sizeof(MpcPw):
             raise RuntimeError("mpc_pw layout mismatch between library and binding")
+        if lib().mpc_sizeof_fno_col() != C.sizeof(MpcFnoCol):
+            raise RuntimeError("mpc_fno_col layout mismatch between library and binding")
         self.ws = DArr((1 << 22,))                # split-K workspace (16 MiB)
         self.gemm_flops = 0                       # 2 M N K summed over the matrix-core products issued
 
@@ -168,6 +178,36 @@ class Ops:
         a.out = _ptr(out)
         a.act = 1 if act else 0
         check(lib().mpc_fno_pointwise(C.cast(C.pointer(a), C.c_void_p), _stream()), "mpc_fno_pointwise")
+
+    def dft(self, G, src, dst, nslice, m, kk, nb, h, sign, bwd=False):
+        """dst = the truncated complex DFT G = [cos; sin] (2m x kk) of every slice of src, recombined (bwd: its
+        transpose)"""
+        self.gemm_flops += 2 * 2 * m * kk * nb * 2 * h * nslice
+        check(lib().mpc_fno_dft(_ptr(G), _ptr(src), _ptr(dst), nslice, m, kk, nb, h, sign, 1 if bwd else 0,
+                                _stream()), "mpc_fno_dft")
+
+    def pack(self, G, kind, m, kk):
+        """a constant matrix as the fused kernels read it (mpc_fno_pack)"""
+        n = lib().mpc_fno_pack_bytes(kind, m, kk)
+        check(n if n < 0 else 0, "mpc_fno_pack_bytes")
+        d = DArr(((n + 3) // 4,))
+        check(lib().mpc_fno_pack(_ptr(G), _ptr(d), kind, m, kk, _stream()), "mpc_fno_pack")
+        return d
+
+    def column(self, nb, width, npos, nt, n2, v, v_bs, w, bias, V6=None, Gt=None, Ft=None, act=False, zs=None,
+               out=None, C1=None, head=None):
+        """the work of every transverse point between two layers' transverse transforms (mpc_fno_column);
+        head: (hidden, Q1, q1, Q2, q2, x, x batch stride, y)"""
+        a = MpcFnoCol()
+        a.nb, a.width, a.npos, a.nt, a.n2, a.act = nb, width, npos, nt, n2, 1 if act else 0
+        a.v, a.v_bs, a.w, a.bias = _ptr(v), v_bs, _ptr(w), _ptr(bias)
+        for name, d in (("V6", V6), ("Gt", Gt), ("Ft", Ft), ("zs", zs), ("out", out), ("C1", C1)):
+            setattr(a, name, _ptr(d) if d is not None else None)
+        if head is not None:
+            a.h, a.x_bs = head[0], head[6]
+            a.q1w, a.q1, a.q2w, a.q2, a.x, a.y = (_ptr(d) for d in head[1:6] + head[7:8])
+        self.gemm_flops += 2 * nb * width * npos * nt * n2 * ((V6 is not None) + (C1 is not None))
+        check(lib().mpc_fno_column(C.cast(C.pointer(a), C.c_void_p), _stream()), "mpc_fno_column")
 
     def transpose(self, src, dst, rows, cols):
         check(lib().mpc_fno_transpose(_ptr(src), _ptr(dst), rows, cols, _stream()), "mpc_fno_transpose")
@@ -288,6 +328,13 @@ class FnoGpu:
         self.m = {k: zeros(v.shape) for k, v in self.p.items()}
         self.v = {k: zeros(v.shape) for k, v in self.p.items()}
         self.mats = {k: DArr.of(v) for k, v in dft_mats(cfg).items()}
+        self.fused = self._fits()
+        self.packed = {}
+        if self.fused:
+            n2 = 2 * cfg.mt
+            for name, kind, m, k in (("Gyf", 0, cfg.my, cfg.Y), ("Gxf", 0, cfg.mx, cfg.X), ("Gxi", 0, cfg.X, cfg.mx),
+                                     ("Gyi", 0, cfg.Y, cfg.my), ("Gt", 2, n2, cfg.T), ("Ft", 3, cfg.T, n2)):
+                self.packed[name, kind] = self.ops.pack(self.mats[name], kind, m, k)
         self.step = 0
         self._buf = {}
 
@@ -402,8 +449,67 @@ class FnoGpu:
                           offA=b * nout * npts, offB=b * nin * npts)
 
     # ---- network ---------------------------------------------------------------
+    def _fits(self):
+        """whether the fused kernels take this network's sizes (they hold a whole t-line of every channel in a
+        workgroup); larger ones run the separate kernels"""
+        c, L = self.cfg, lib()
+        return bool(c.cout == 2 and L.mpc_fno_column_fits(c.width, c.cin, c.T, 2 * c.mt, c.hidden) and
+                    all(L.mpc_fno_dft_fits(m, k, bwd) for bwd in (0, 1)
+                        for m, k in ((c.my, c.Y), (c.mx, c.X), (c.X, c.mx), (c.Y, c.my))))
+
+    def _modes_fwd(self, C1, l, V6, save, B):
+        """V6 = the layer's mode path of its t-DFT C1: forward y and x transforms, per-mode mixing, inverse x and y"""
+        c, o, M = self.cfg, self.ops, self.packed
+        W, X, Y, mx, my, mt = c.width, c.X, c.Y, c.mx, c.my, c.mt
+        n2 = 2 * mt
+        V2 = self._b("V2", (B * W * X, my, n2))
+        o.dft(M["Gyf", 0], C1, V2, B * W * X, my, Y, 1, mt, -1)
+        V3 = save if save is not None else self._b("V3", (B, W, mx, my, n2))
+        o.dft(M["Gxf", 0], V2, V3, B * W, mx, X, my, mt, -1)
+        U = self._b("U", (B, W, mx, my, n2))
+        self._mix(V3, self.p[f"Rr{l}"], self.p[f"Ri{l}"], U, B)
+        V5 = self._b("V5", (B * W, X, my, n2))
+        o.dft(M["Gxi", 0], U, V5, B * W, X, mx, my, mt, +1)
+        o.dft(M["Gyi", 0], V5, V6, B * W * X, Y, my, 1, mt, +1)
+
+    def _forward_fused(self, x, keep):
+        c, o, M = self.cfg, self.ops, self.packed
+        B, W, H, npos = x.shape[0], c.width, c.hidden, c.X * c.Y
+        npts, n2 = npos * c.T, 2 * c.mt
+        st = {"x": x}
+        shp = (B, W, c.X, c.Y, c.T)
+        C1, V6 = self._b("C1", (B * W * npos, n2)), self._b("V6", (B * W * npos, n2))
+        y = self._b("y", (B, c.cout, c.X, c.Y, c.T))
+        v = self._b("v0", shp)
+        o.column(B, W, npos, c.T, n2, x, c.cin * npts, self.p["P"], self.p["bP"], Ft=M["Ft", 3], out=v, C1=C1)
+        for l in range(c.layers):
+            last = l == c.layers - 1
+            V3 = self._b(f"V3{l}", (B, W, c.mx, c.my, n2)) if keep else None
+            self._modes_fwd(C1, l, V6, V3, B)
+            args = (B, W, npos, c.T, n2, v, W * npts, self.p[f"W{l}"], self.p[f"b{l}"], V6, M["Gt", 2], M["Ft", 3])
+            if last and not keep:
+                o.column(*args, head=(H, self.p["Q1"], self.p["q1"], self.p["Q2"], self.p["q2"], x, c.cin * npts, y))
+                return y
+            z = self._b(f"z{l}", shp) if keep and not last else None
+            # in place without keep (a point's channels are read before they are
+            # written): one activation buffer and the mode rows fit the last-level cache
+            vn = self._b(f"v{l + 1}", shp) if keep else v
+            o.column(*args, act=not last, zs=z, out=vn, C1=C1)
+            if keep:
+                st[f"v{l}"], st[f"z{l}"], st[f"V3{l}"] = v, z, V3
+            v = vn
+        hz, h = self._b("hz", (B, H, c.X, c.Y, c.T)), self._b("h", (B, H, c.X, c.Y, c.T))
+        o.pointwise(v, W, self.p["Q1"], W, 1, h, H, B, npts, bias=self.p["q1"], zs=hz, act=True)
+        o.pointwise(h, H, self.p["Q2"], H, 1, y, c.cout, B, npts, bias=self.p["q2"], zin=x, beta=1.0,
+                    zin_bs=c.cin * npts)
+        st["vL"], st["hz"], st["h"] = v, hz, h
+        self._st = st
+        return y
+
     def forward(self, x, keep=False):
         """x: (B, cin, X, Y, T) float32 cuda -> pred (B, cout, X, Y, T).  keep: save activations for backward"""
+        if self.fused:
+            return self._forward_fused(x, keep)
         c = self.cfg
         B = x.shape[0]
         npts = c.X * c.Y * c.T
@@ -460,7 +566,7 @@ class FnoGpu:
         for l in reversed(range(c.layers)):
             act = l < c.layers - 1
             dz = self._b("dz", dv.shape)
-            o.act_bwd(st[f"z{l}"], dv, dz, act)
+            o.act_bwd(st[f"z{l}"] if act else dv, dv, dz, act)
             o.bias_grad(dz, self.g[f"b{l}"], B, W, npts)
             self._pw_bwd_weight(dz, st[f"v{l}"], self.g[f"W{l}"], W, W, npts, B)
             self._pw_bwd_input(self.p[f"W{l}"], dz, dv, W, W, npts, B)

@@ -281,3 +281,45 @@ def test_configured_network_matches_cpu_network(gpu_lib):
         rel = abs(an - fd) / max(abs(fd), scale, 1e-12)
         print(f"  {label}: loss gpu {loss_gpu:.6f} fd {fd:+.6e} gpu {an:+.6e} rel {rel:.2e}", flush=True)
         assert rel <= 5e-2, label
+
+
+@pytest.mark.parametrize("W,B,X,Y,T,mx,my,mt,H", [
+    # one t tile, two points a group and an odd point count; the longest line and the most mode columns
+    (8, 1, 5, 3, 7, 2, 2, 3, 16), (32, 2, 6, 5, 256, 4, 4, 32, 64),
+    # ragged tiles on both sides of the two-points rule, mode columns that fill no tile
+    (16, 3, 9, 7, 129, 6, 4, 9, 32), (64, 1, 8, 9, 128, 8, 6, 17, 64), (32, 1, 64, 3, 33, 34, 2, 16, 8),
+    # transverse lengths at and past a step of the matrix products
+    (16, 2, 16, 33, 225, 16, 18, 25, 32)])
+def test_fused_layers_match_separate_kernels(gpu_lib, W, B, X, Y, T, mx, my, mt, H):
+    """the fused column and DFT kernels against the separate GEMM,
+    recombination and pointwise kernels on the same network: the same
+    operands, roundings and summation order, so with activations kept every
+    saved tensor and the prediction are the same bits.  Without, GELU is formed
+    in another way (both forms are within 3 ulp of 0.5 |x| (1 + |erf|)) and the
+    head adds its channels in another order; a BF16 operand of a later layer
+    that rounds the other way moves by 2^-8, and one in 1e4 does: 1e-4 of the
+    change the network makes"""
+    from mpc_amd.fno import FnoConfig, FnoGpu, init_params
+    print(f"case fused W={W} B={B} X={X} Y={Y} T={T} modes={mx},{my},{mt} H={H}", flush=True)
+    cfg = FnoConfig(X=X, Y=Y, T=T, width=W, layers=2, mx=mx, my=my, mt=mt, hidden=H)
+    p = init_params(cfg, seed=W + T)
+    rng = np.random.default_rng(T)
+    for k in p:
+        if k[0] == "R":
+            p[k] *= W
+        if k[0] in "bq":
+            p[k] = 0.1 * rng.standard_normal(p[k].shape)
+    x = rng.standard_normal((B, cfg.cin, X, Y, T)).astype(np.float32)
+    net = FnoGpu(cfg, p)
+    assert net.fused
+    got = {}
+    for fused in (True, False):
+        net.fused = fused
+        y = net.forward(_t(x)).numpy()
+        yk = net.forward(_t(x), keep=True).numpy()
+        got[fused] = (y, yk, net._st["v1"].numpy(), net._st["z0"].numpy(), net._st["V31"].numpy(),
+                      net._st["vL"].numpy())
+    for a, b in zip(got[True][1:], got[False][1:]):
+        assert np.array_equal(a, b)
+    a, b = got[True][0].astype(np.float64), got[False][0].astype(np.float64)
+    assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b - x[:, :2])
