@@ -139,7 +139,7 @@ template <class T> static int setup_tables(mpc_ctx *c) {
     RCHK(upload_vec(&c->tw_t, twiddles<T>(c->nt)));
     RCHK(upload_vec(&c->tw_x, twiddles<T>(c->nx)));
     std::vector<T> wf(c->nt);
-    for (int k = 0; k < c->nt; k++) wf[k] = (T)c->w[(k + c->nt / 2) % c->nt]; /* propagation.c:170-177 */
+    for (int k = 0; k < c->nt; k++) wf[k] = (T)c->w[(t_order(c->nt, k) + c->nt / 2) % c->nt]; /* propagation.c:170-177 */
     RCHK(upload_vec(&c->wfft, wf));
     /* mirror: curvature phase (FP64, reduced) x hard aperture x sqrt(Ab_M) */
     std::vector<cx<T>> M((size_t)c->nx * c->ny);
@@ -247,7 +247,7 @@ extern "C" long long mpc_field_bytes(mpc_ctx *c) { return c ? (long long)c->esz 
 /* ------------------------------------------------------------------------ */
 /* tables                                                                    */
 /* ------------------------------------------------------------------------ */
-/* kind 't': exp(ct (i beta_k - alpha/2)) / Nt, beta in FFT order
+/* kind 't': exp(ct (i beta_k - alpha/2)) / Nt, beta in the field's frequency order (t_order)
  *           (propagation.c:150-156 for one half step, ct = dz/2);
  * kind 'x'/'y': exp(-i c k^2 / (2 k0)) / n, k in FFT order, c = sum of
  *           s * dz/2 over the merged half steps (conj of calcexpR). */
@@ -263,7 +263,7 @@ template <class T> static const cx<T> *get_table(mpc_ctx *c, char kind, double c
         const int nt = c->nt;
         tab.resize(nt);
         for (int k = 0; k < nt; k++) {
-            const double beta = c->betas[(k + nt / 2) % nt];
+            const double beta = c->betas[(t_order(nt, k) + nt / 2) % nt];
             const double mag = std::exp(-c->p.alpha / 2.0 * coef) / (kind == 't' ? nt : 1);
             const double ph = reduce_2pi(beta * coef);
             tab[k] = mk((T)(mag * std::cos(ph)), (T)(mag * std::sin(ph)));
@@ -287,7 +287,10 @@ template <class T> static const cx<T> *get_table(mpc_ctx *c, char kind, double c
 template <class T> static const cx<T> *user_table(mpc_ctx *c, const char *tag, const cufftDoubleComplex *src,
                                                   int n, double scale, bool conj) {
     std::vector<cx<T>> tab(n);
-    for (int i = 0; i < n; i++) tab[i] = mk((T)(src[i].x * scale), (T)((conj ? -src[i].y : src[i].y) * scale));
+    for (int i = 0; i < n; i++) {
+        const cufftDoubleComplex &e = src[tag[0] == 't' ? t_order(n, i) : i];   /* FFT order to the field's */
+        tab[i] = mk((T)(e.x * scale), (T)((conj ? -e.y : e.y) * scale));
+    }
     std::string key = std::string("u:") + tag;
     auto it = c->tables.find(key);
     if (it != c->tables.end()) { (void)hipFree(it->second); c->tables.erase(it); }

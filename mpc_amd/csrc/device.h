@@ -81,17 +81,138 @@ __device__ __forceinline__ void line_fft(cx<T> (&v)[PL::E], int tid, cx<T> *lds,
     DevFftP<T, N, PL::E, DIR, PAD, BOFF, typename PL::R>::run(v, tid, lds, ls, tw);
 }
 
-/* t-line geometry: plan, LDS layout (XOR swizzle keyed to E) and lines per
- * 256-thread block */
+/*
+ * A wait for the other threads of a t-line: within one wavefront (WAVE) its
+ * LDS operations complete in order, so it only keeps the compiler from moving
+ * them across; otherwise the workgroup's barrier.
+ */
+template <bool WAVE> __device__ __forceinline__ void line_sync() {
+    if constexpr (WAVE) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        __syncthreads();
+    }
+}
+
+/* t-line geometry: plan and lines per 256-thread block.  WN points are one wavefront's transform (or half of
+ * one's at 256 points); WAVE: a line lies within a wavefront, so its
+ * workgroup has no barriers and its wavefronts run independently. */
 template <int NT_, class PL_ = TPlan<NT_>> struct TGeo {
     static constexpr int NT = NT_;
     using PL = PL_;
     static constexpr int E = PL::E, TPL = NT / E;
     static constexpr int LPB = (256 / TPL) > 0 ? (256 / TPL) : 1;
     static constexpr int THREADS = LPB * TPL;
-    static constexpr int PAD = -ilog2(E);              /* XOR swizzle, see padi */
-    static constexpr int FFT_ELEMS = padded_elems<PAD>(NT);
+    static constexpr int WN = t_wave_len(NT), R1 = NT / WN;
+    static constexpr bool WAVE = R1 == 1;
 };
+
+/* the wavefront part of a t-line transform: Stockham stages over the WN
+ * elements of one region, twiddles from the NT-point table or cached */
+template <class T, int NT, int WN, int E, int DIR, int Ns, int R, int... Rest> struct WaveFft {
+    static __device__ __forceinline__ void next(cx<T> (&v)[E], int lane, cx<T> *reg) {
+        WaveX<T, WN>::template put<Ns>(v, lane, reg);
+        line_sync<true>();
+        WaveX<T, WN>::template get<Ns>(v, lane, reg);
+        line_sync<true>();
+    }
+    static __device__ __forceinline__ void run(cx<T> (&v)[E], int lane, cx<T> *reg, const cx<T> *tw) {
+        fft_stage_t<T, WN, E, R, Ns, DIR, true, 0>(v, lane, reg, 1, TwFromTable<T, WN, R, Ns, DIR, NT / WN>{tw});
+        if constexpr (sizeof...(Rest) != 0) {
+            next(v, lane, reg);
+            WaveFft<T, NT, WN, E, DIR, Ns * R, Rest...>::run(v, lane, reg, tw);
+        }
+    }
+    static __device__ __forceinline__ void run(cx<T> (&v)[E], int lane, cx<T> *reg,
+                                               const TwChain<T, WN, E, Ns, R, Rest...> &ch) {
+        fft_stage_t<T, WN, E, R, Ns, DIR, true, 0>(v, lane, reg, 1, TwFromPowers<T, R, E / R, DIR>{ch.p});
+        if constexpr (sizeof...(Rest) != 0) {
+            next(v, lane, reg);
+            WaveFft<T, NT, WN, E, DIR, Ns * R, Rest...>::run(v, lane, reg, ch.next);
+        }
+    }
+};
+template <class T, class G, class Rad> struct TLineP;
+/*
+ * The transform of one t-line.  In the Stockham form over the workgroup, with
+ * XOR-swizzled exchanges, the FP32 t-line was bound by VALU instructions (at
+ * 2048 points 226 per point; VALU busy 94%), of which addresses were over a
+ * quarter; FP64 by the exchanges' barriers.  With wavefront-level transforms,
+ * pitched exchanges and the small-step exponential it is 205 per point and
+ * one barrier a transform instead of six: 256x256x2048 1202 -> 1102 us (FP32),
+ * 2160 -> 1850 (FP64), 128x128x512 80 -> 60, 64x64x256 17.2 -> 14.9.
+ */
+template <class T, class G, int... Rs> struct TLineP<T, G, Radices<Rs...>> {
+    static constexpr int E = G::E, WN = G::WN, R1 = G::R1;
+    static constexpr int REGION = WaveX<T, WN>::ELEMS, ELEMS = R1 * REGION;   /* of a line's exchange buffer */
+    /* a thread's twiddle powers of every stage, loaded once per kernel */
+    struct Chain {
+        TCross<T, G::NT, R1 == 1 ? 2 : R1, E> x;
+        TwChain<T, WN, E, 1, Rs...> w;
+        __device__ __forceinline__ void load(const cx<T> *tw, int tid) {
+            if constexpr (R1 > 1) x.load(tw, tid);
+            w.load(tw, tid % (WN / E), R1);
+        }
+    };
+    /*
+     * The line's transform (DIR -1: time to frequency).  lds: the line's
+     * exchange buffer; BOFF != 0: a second one BOFF elements on, and the
+     * calls alternate between them (par), so a transform writes where no
+     * slower wavefront can still be reading the one before, and one barrier
+     * (between the writes and the reads of the step across wavefronts)
+     * suffices.
+     */
+    template <int DIR, int BOFF, class Tw>
+    static __device__ __forceinline__ void run(cx<T> (&v)[E], int tid, cx<T> *lds, int &par, const Tw &tw) {
+        constexpr bool TABLE = std::is_pointer_v<Tw>;
+        using WF = WaveFft<T, G::NT, WN, E, DIR, 1, Rs...>;
+        auto wave_part = [&](int lane, cx<T> *reg) {
+            if constexpr (TABLE) WF::run(v, lane, reg, tw);
+            else WF::run(v, lane, reg, tw.w);
+        };
+        if constexpr (R1 == 1) {
+            line_sync<true>();
+            wave_part(tid, lds);
+            line_sync<true>();
+        } else {
+            if constexpr (BOFF != 0) {
+                lds += par ? BOFF : 0;
+                par ^= 1;
+            } else {
+                __syncthreads();
+            }
+            cx<T> *reg = lds + tid / 64 * REGION;
+            const int lane = tid % 64;
+            auto cross = [&](auto &&f) {
+                if constexpr (TABLE) {
+                    TCross<T, G::NT, R1, E> x;
+                    x.load(tw, tid);
+                    f(x);
+                } else {
+                    f(tw.x);
+                }
+            };
+            if constexpr (DIR < 0) {
+                cross([&](const auto &x) { x.fwd(v, tid, lds); });
+                __syncthreads();
+#pragma unroll
+                for (int m = 0; m < E; ++m) v[m] = reg[lane + 64 * m];
+                line_sync<true>();
+                wave_part(lane, reg);
+            } else {
+                line_sync<true>();
+                wave_part(lane, reg);
+                line_sync<true>();
+#pragma unroll
+                for (int m = 0; m < E; ++m) reg[lane + 64 * m] = v[m];
+                __syncthreads();
+                cross([&](const auto &x) { x.inv(v, tid, lds); });
+            }
+        }
+    }
+};
+template <class T, class G> using TLine = TLineP<T, G, typename TPlan<G::WN>::R>;
 
 /* ---------------------------------------------------------------------- */
 /* plasma model pieces (FP64 in both precisions)                           */
@@ -168,15 +289,17 @@ __device__ __forceinline__ double one_minus_exp_neg(double R) {
     return -expm1(-R);
 }
 
-/* plasma arrays: the exchange buffers' swizzle, so both the per-element
- * accesses (unit lane stride) and the scan's per-thread segments (lane
- * stride E) are free of bank conflicts */
-template <class G> __device__ __forceinline__ int padp(int i) { return padi<G::PAD>(i); }
-/* the swizzled position of element tid + TPL*m (constant offsets where the
- * layout allows, see padi_strided) */
+/* plasma arrays: element k in row k % 8, column k / 8 of a pitched array, so
+ * that the per-element accesses (k = tid + TPL m) and the scan's per-thread
+ * segments (k = 8 tid + i) both take one base address, constant offsets and
+ * no bank conflicts (rows step by 2 elements of 8 bytes) */
+template <class G> constexpr int PLANE = G::TPL + 2;
+template <class G> __device__ __forceinline__ int padp(int k) { return k % 8 * PLANE<G> + k / 8; }
 template <class G> __device__ __forceinline__ int padp_tm(int tid, int m) {
-    return padi_strided<G::PAD, G::NT / G::E>(tid, m);
+    return tid % 8 * PLANE<G> + tid / 8 + G::TPL / 8 * m;
 }
+/* element 8 tid + i of the scan's walks */
+template <class G> __device__ __forceinline__ int padp_seg(int tid, int i) { return i * PLANE<G> + tid; }
 
 /*
  * Lane moves within a wavefront by DPP (no LDS round trip): CTRL is
@@ -233,12 +356,13 @@ __device__ __forceinline__ void affine_combine(double &gm, double &gc, double &g
 }
 
 /*
- * Reverse-t affine scan over one line.  Element k carries the map
- * f_k(R) = m_k R + c_k, given by coef(k, m_k, c_k); the result
- * R_k = f_k(R_{k+1}), R_NT = 0, is handed to out(k, R_k).  Thread tid owns the
- * consecutive segment [tid*E, tid*E + E): segment maps are composed serially,
+ * Reverse-t affine scan over one line.  Thread tid owns the consecutive
+ * segment of elements k = tid*E + i, i < E.  Element k carries the map
+ * f_k(R) = m_k R + c_k, given by coef(i, m_k, c_k); the result
+ * R_k = f_k(R_{k+1}), R_NT = 0, is handed to out(i, R_k).  Segment maps are composed serially,
  * combined across lanes with a shuffle-based suffix scan and across wavefronts
- * through LDS (scr, 3 NW + TPL doubles), then each thread re-walks its
+ * through LDS (scr, 3 NW + TPL doubles; not used by lines within a wavefront),
+ * then each thread re-walks its
  * segment from the suffix value of the segments after it.  The carries of
  * the lane and wavefront combines are compensated (affine_combine); the
  * suffix value is rounded once, where a thread's walk starts.  coef must give
@@ -250,29 +374,35 @@ __device__ __forceinline__ bool affine_suffix_scan(int tid, double *scr, Coef co
     constexpr int E = G::E, TPL = G::NT / E;
     constexpr int W = TPL < 64 ? TPL : 64;
     constexpr int NW = (TPL + 63) / 64;
-    const int lo = tid * E;
     double gm = 1.0, gc = 0.0, gl = 0.0, cs = gate_init;
 #pragma unroll
     for (int i = E - 1; i >= 0; --i) {
         double mk, ck;
-        coef(lo + i, mk, ck);
+        coef(i, mk, ck);
         gc = mk * gc + ck;
         gm = mk * gm;
         if constexpr (GATED) cs += ck;
     }
     if constexpr (GATED) {
         /* the line's sum of c_k (plus gate_init of every thread) goes to
-         * gate(); when it returns true on every line of the workgroup the
-         * scan stops here and returns false (out is not called) */
-        double *part = scr + 3 * NW + TPL;                 /* NW doubles */
+         * gate(); when it returns true on every line of the workgroup (of the
+         * wavefront, where lines lie within one) the scan stops here and
+         * returns false (out is not called) */
         lanes_sum<W>(cs);
-        if ((tid % W) == (W == 64 ? 63 : 0)) part[tid / W] = cs;
-        __syncthreads();
         double sum = 0.0;
+        if constexpr (G::WAVE) {
+            sum = W == 64 ? __shfl(cs, 63) : cs;
+        } else {
+            double *part = scr + 3 * NW + TPL;             /* NW doubles */
+            if (tid % 64 == 63) part[tid / 64] = cs;
+            __syncthreads();
 #pragma unroll
-        for (int w = 0; w < NW; ++w) sum += part[w];
+            for (int w = 0; w < NW; ++w) sum += part[w];
+        }
         bool stop = gate(sum);
-        if constexpr (G::LPB > 1) {
+        if constexpr (G::WAVE) {
+            stop = __all(stop);
+        } else if constexpr (G::LPB > 1) {
             stop = !__syncthreads_or(!stop);                /* whole workgroup or none */
         } else {
             stop = __builtin_amdgcn_readfirstlane((int)stop);   /* the same on every lane */
@@ -287,23 +417,28 @@ __device__ __forceinline__ bool affine_suffix_scan(int tid, double *scr, Coef co
         const double ol = __shfl_down(gl, d, W);
         if (lane + d < W) affine_combine(gm, gc, gl, om, oc, ol);
     }
-    if constexpr (NW > 1) {
+    double R;                                              /* the suffix value of the segments after this thread's */
+    if constexpr (G::WAVE) {
+        const double next = __shfl_down(gc + gl, 1, W);
+        R = lane + 1 < W ? next : 0.0;
+        line_sync<true>();
+    } else {
         const int wv = tid / 64;
         if (lane == 0) { scr[3 * wv] = gm; scr[3 * wv + 1] = gc; scr[3 * wv + 2] = gl; }
         __syncthreads();
         for (int w2 = wv + 1; w2 < NW; ++w2) affine_combine(gm, gc, gl, scr[3 * w2], scr[3 * w2 + 1], scr[3 * w2 + 2]);
+        scr[3 * NW + tid] = gc + gl;
+        __syncthreads();
+        R = (tid + 1 < TPL) ? scr[3 * NW + tid + 1] : 0.0;
     }
-    scr[3 * NW + tid] = gc + gl;
-    __syncthreads();
-    double R = (tid + 1 < TPL) ? scr[3 * NW + tid + 1] : 0.0;
 #pragma unroll
     for (int i = E - 1; i >= 0; --i) {
         double mk, ck;
-        coef(lo + i, mk, ck);
+        coef(i, mk, ck);
         R = mk * R + ck;
-        out(lo + i, R);
+        out(i, R);
     }
-    __syncthreads();
+    line_sync<G::WAVE>();
     return true;
 }
 
@@ -313,10 +448,11 @@ __device__ __forceinline__ bool affine_suffix_scan(int tid, double *scr, Coef co
  * for the result */
 template <class G, class T> struct PlasmaLds {
     static constexpr int NT = G::NT, E = G::E, TPL = NT / E, NW = (TPL + 63) / 64;
-    static constexpr int ARR = padded_elems<G::PAD>(NT);   /* elements per array */
+    static constexpr int ARR = 8 * PLANE<G>;               /* elements per array */
+    static_assert(E == 8, "the plasma arrays have a row per element of a thread");
     static constexpr int SCR = 3 * NW + TPL + NW;           /* doubles: the scan's scratch, then the
                                                                cold-line test's per-wave partials */
-    static constexpr int SVB = 2 * ARR * (int)sizeof(T);
+    static constexpr int SVB = 2 * NT * (int)sizeof(T);
     static constexpr bool SV = G::LPB * ((2 * ARR + SCR) * 8 + SVB) <= 80 * 1024;
     static constexpr int BYTES = (2 * ARR + SCR) * 8 + (SV ? SVB : 0);
 };
@@ -431,10 +567,10 @@ __device__ __forceinline__ void plasma_line(const cx<T> (&A)[G::E], int tid, dou
     constexpr int NT = G::NT;
     constexpr int E = L::E, TPL = L::TPL;
     double *U = lds, *X = lds + L::ARR, *scr = lds + 2 * L::ARR;
-    T *S = reinterpret_cast<T *>(lds + 2 * L::ARR + L::SCR), *V = S + L::ARR;   /* used when L::SV */
+    T *S = reinterpret_cast<T *>(lds + 2 * L::ARR + L::SCR), *V = S + NT;   /* used when L::SV; element tid + TPL m there */
     int anyc = 0;
     T invs[L::SV ? 1 : E];
-    __syncthreads();              /* the LDS may still be read by the caller's last exchange */
+    line_sync<G::WAVE>();         /* the LDS may still be read by the caller's last exchange */
 #pragma unroll
     for (int m = 0; m < E; ++m) {
         const int k = padp_tm<G>(tid, m);                  /* element tid + TPL*m, swizzled */
@@ -447,8 +583,8 @@ __device__ __forceinline__ void plasma_line(const cx<T> (&A)[G::E], int tid, dou
         U[k] = 1.0 - a;
         X[k] = b * (1.0 - a) + a;
         if constexpr (L::SV) {
-            S[k] = sig;
-            V[k] = pe.inv_s;
+            S[tid + TPL * m] = sig;
+            V[tid + TPL * m] = pe.inv_s;
         } else {
             invs[m] = pe.inv_s;
         }
@@ -461,10 +597,10 @@ __device__ __forceinline__ void plasma_line(const cx<T> (&A)[G::E], int tid, dou
         } else {
             pe.I = 0.0;
         }
-        pe.inv_s = L::SV ? V[padp_tm<G>(tid, m)] : invs[L::SV ? 0 : m];
+        pe.inv_s = L::SV ? V[tid + TPL * m] : invs[L::SV ? 0 : m];
         return pe;
     };
-    __syncthreads();
+    line_sync<G::WAVE>();
     /* U <- u = 1 - exp(-R); a cold line (COLD) stops after the sum of X */
     double s_line = 0.0;
     double s_lim = 0.0;
@@ -475,29 +611,30 @@ __device__ __forceinline__ void plasma_line(const cx<T> (&A)[G::E], int tid, dou
         s_lim = fmin(ColdLine<T>::S_MAX, ColdLine<T>::EPS / (pk.rho_nt * dz_abs * pk.sig_bound));
     }
     const bool scanned = affine_suffix_scan<G, COLD>(tid, scr,
-        [&](int k, double &mk, double &ck) { mk = U[padp<G>(k)]; ck = X[padp<G>(k)]; },
-        [&](int k, double R) { U[padp<G>(k)] = one_minus_exp_neg(R); },
+        [&](int i, double &mk, double &ck) { mk = U[padp_seg<G>(tid, i)]; ck = X[padp_seg<G>(tid, i)]; },
+        [&](int i, double R) { U[padp_seg<G>(tid, i)] = one_minus_exp_neg(R); },
         anyc ? __builtin_inf() : 0.0,                      /* a second species: never cold */
         [&](double sum) { s_line = sum; return sum <= s_lim; });
     if (!scanned) {
         rho_max = fmax(rho_max, s_line);
-        __syncthreads();          /* the caller's next exchange overwrites this LDS */
+        line_sync<G::WAVE>();     /* the caller's next exchange overwrites this LDS */
         return;
     }
-    const int block_anyc = __syncthreads_or(anyc);
+    const int block_anyc = G::WAVE ? __any(anyc) : __syncthreads_or(anyc);
     if (block_anyc) {
 #pragma unroll
         for (int m = 0; m < E; ++m) X[padp_tm<G>(tid, m)] = elem(m).adk_b(pk, 2);
-        __syncthreads();
+        line_sync<G::WAVE>();
         /* X <- ions2: m_k = 1 - c_k, c'_k = c_k u_{k+1} */
         affine_suffix_scan<G>(tid, scr,
-            [&](int k, double &mk, double &ck) {
-                const double c = X[padp<G>(k)];
+            [&](int i, double &mk, double &ck) {
+                const int k = E * tid + i;
+                const double c = X[padp_seg<G>(tid, i)];
                 const double un = (k + 1 < NT) ? U[padp<G>(k + 1)] : 0.0;
                 mk = 1.0 - c;
                 ck = c * un;
             },
-            [&](int k, double R) { X[padp<G>(k)] = R; });
+            [&](int i, double R) { X[padp_seg<G>(tid, i)] = R; });
     }
 #pragma unroll
     for (int m = 0; m < E; ++m) {
@@ -507,29 +644,30 @@ __device__ __forceinline__ void plasma_line(const cx<T> (&A)[G::E], int tid, dou
         const double fr = i1 + 2.0 * i2;
         T tc, sig;
         if constexpr (L::SV) {
-            sig = S[k];
-            tc = (T)pk.kt * V[k];
+            sig = S[tid + TPL * m];
+            tc = (T)pk.kt * V[tid + TPL * m];
         } else {
             sig = elem(m).sigma(pk, &tc);
         }
         rho_max = fmax(rho_max, fr);
         sink(m, (T)fr * sig, tc);
     }
-    __syncthreads();
+    line_sync<G::WAVE>();
 }
 
 /* ---------------------------------------------------------------------- */
 /* t-line kernel                                                           */
 /* ---------------------------------------------------------------------- */
-/* per-line LDS: the FFT exchange buffer (doubled, BOFF != 0, while a
- * workgroup's LDS stays within 80 KB, i.e. two workgroups per CU) unioned
+/* per-line LDS: the FFT exchange buffer (doubled, BOFF != 0, where a line
+ * spans wavefronts and while a workgroup's LDS stays within 80 KB, i.e. two
+ * workgroups per CU) unioned
  * with the plasma arrays */
 template <class T, class G, bool PLASMA> struct TCfg {
     static constexpr int E = G::E, TPL = G::TPL, LPB = G::LPB, THREADS = G::THREADS;
-    static constexpr int FFT1 = G::FFT_ELEMS * (int)sizeof(cx<T>);
+    static constexpr int FFT1 = TLine<T, G>::ELEMS * (int)sizeof(cx<T>);
     static constexpr int PL_BYTES = PLASMA ? PlasmaLds<G, T>::BYTES : 0;
-    static constexpr bool DB = LPB * 2 * FFT1 <= 80 * 1024;
-    static constexpr int BOFF = DB ? G::FFT_ELEMS : 0;
+    static constexpr bool DB = !G::WAVE && LPB * 2 * FFT1 <= 80 * 1024;
+    static constexpr int BOFF = DB ? TLine<T, G>::ELEMS : 0;
     static constexpr int FFT_BYTES = (DB ? 2 : 1) * FFT1;
     static constexpr int LINE_BYTES = ((FFT_BYTES > PL_BYTES ? FFT_BYTES : PL_BYTES) + 15) / 16 * 16;
     static_assert(LPB * LINE_BYTES <= 160 * 1024, "t-line workgroup exceeds the LDS");
@@ -619,6 +757,49 @@ template <class T> __device__ __forceinline__ T exp_t(T x);
 template <> __device__ __forceinline__ double exp_t<double>(double x) { return exp(x); }
 template <> __device__ __forceinline__ float exp_t<float>(float x) { return expf(x); }
 
+/*
+ * exp(x.re), sin and cos(x.im) of a small nonlinear step: |re| < RE and |im| <
+ * IM, which a wavefront's steps usually are (a whole pass turns the phase by a
+ * few radians over hundreds of steps).  Taylor polynomials whose truncation
+ * is below 2^-26 (FP32) and 2^-55 (FP64) relative: exp to x^4 / x^7, sin to
+ * x^5 / x^9, cos to x^6 / x^10.  Taken for all of a thread's elements at once:
+ * checked element by element, the general forms below cost 59 instead of 19
+ * instructions per point in FP32 (of 242 of the whole t-line).
+ */
+template <class T> struct SmallStep { static constexpr T RE = (T)0.03125, IM = (T)0.125; };
+__device__ __forceinline__ float max_abs(float m, float x) { return fmaxf(m, fabsf(x)); }
+__device__ __forceinline__ double max_abs(double m, double x) { return fmax(m, fabs(x)); }
+__device__ __forceinline__ void small_exp(cx<float> x, float &e, float &s, float &c) {
+    float p = fmaf(x.re, 1.0f / 24.0f, 1.0f / 6.0f);
+    p = fmaf(p, x.re, 0.5f);
+    p = fmaf(p, x.re, 1.0f);
+    e = fmaf(p, x.re, 1.0f);
+    const float r2 = x.im * x.im;
+    s = fmaf(fmaf(r2, 1.0f / 120.0f, -1.0f / 6.0f) * r2, x.im, x.im);
+    p = fmaf(r2, -1.0f / 720.0f, 1.0f / 24.0f);
+    p = fmaf(p, r2, -0.5f);
+    c = fmaf(p, r2, 1.0f);
+}
+__device__ __forceinline__ void small_exp(cx<double> x, double &e, double &s, double &c) {
+    double p = fma(x.re, 1.0 / 5040.0, 1.0 / 720.0);
+    p = fma(p, x.re, 1.0 / 120.0);
+    p = fma(p, x.re, 1.0 / 24.0);
+    p = fma(p, x.re, 1.0 / 6.0);
+    p = fma(p, x.re, 0.5);
+    p = fma(p, x.re, 1.0);
+    e = fma(p, x.re, 1.0);
+    const double r2 = x.im * x.im;
+    p = fma(r2, 1.0 / 362880.0, -1.0 / 5040.0);
+    p = fma(p, r2, 1.0 / 120.0);
+    p = fma(p, r2, -1.0 / 6.0);
+    s = fma(p * r2, x.im, x.im);
+    p = fma(r2, -1.0 / 3628800.0, 1.0 / 40320.0);
+    p = fma(p, r2, -1.0 / 720.0);
+    p = fma(p, r2, 1.0 / 24.0);
+    p = fma(p, r2, -0.5);
+    c = fma(p, r2, 1.0);
+}
+
 /* line FFT with twiddle powers cached per thread (TwChain of the plan) */
 template <class T, int N, int E, int DIR, int PAD, int BOFF, int Ns, int R, int... Rest>
 struct DevFftC {
@@ -662,6 +843,18 @@ __device__ __forceinline__ void opaque_chain(TwChain<T, N, E, Ns, R, Rest...> &c
             for (int i = 0; i < tw_npow<R, T>(); ++i) asm volatile("" : "+v"(ch.p[b][i].re), "+v"(ch.p[b][i].im));
     }
     opaque_chain(ch.next);
+}
+
+template <class C> __device__ __forceinline__ void opaque_line(C &c) {
+    if constexpr (std::is_same_v<C, NoChain>) return;
+    else {
+        opaque_chain(c.w);
+        constexpr int B = sizeof(c.x.p) / sizeof(c.x.p[0]), P = sizeof(c.x.p[0]) / sizeof(c.x.p[0][0]);
+#pragma unroll
+        for (int b = 0; b < B; ++b)
+#pragma unroll
+            for (int i = 0; i < P; ++i) asm volatile("" : "+v"(c.x.p[b][i].re), "+v"(c.x.p[b][i].im));
+    }
 }
 
 /* workgroups resident on the device at once for kernel k (0: unknown) */

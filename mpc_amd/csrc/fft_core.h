@@ -270,10 +270,11 @@ MPC_HD void stage_twiddles(cx<T> (&w)[R], const cx<T> *tw, int idx) {
 }
 
 /* twiddle sources for fft_stage: tw(b, k, w) fills w[R] for butterfly b
- * (of the thread's E/R) whose in-group index is k */
-template <class T, int N, int R, int Ns, int DIR> struct TwFromTable {
+ * (of the thread's E/R) whose in-group index is k; the table is that of an
+ * N * TS-point transform */
+template <class T, int N, int R, int Ns, int DIR, int TS = 1> struct TwFromTable {
     const cx<T> *tw;
-    MPC_HD void operator()(int, int k, cx<T> (&w)[R]) const { stage_twiddles<R, DIR>(w, tw, k * (N / (Ns * R))); }
+    MPC_HD void operator()(int, int k, cx<T> (&w)[R]) const { stage_twiddles<R, DIR>(w, tw, k * (N / (Ns * R)) * TS); }
 };
 template <class T, int R, int B, int DIR> struct TwFromPowers {
     const cx<T> (*p)[(tw_npow<R, T>())];   /* p[b] */
@@ -326,18 +327,19 @@ MPC_HD void fft_stage(cx<T> (&v)[E], int tid, cx<T> *lds, int ls, const cx<T> *t
  * every transform of that length the thread runs, in either direction.
  */
 template <class T, int N, int E, int Ns, int... Rs> struct TwChain {
-    MPC_HD void load(const cx<T> *, int) {}
+    MPC_HD void load(const cx<T> *, int, int = 1) {}
 };
 template <class T, int N, int E, int Ns, int R, int... Rest> struct TwChain<T, N, E, Ns, R, Rest...> {
     static constexpr int B = E / R, NP = tw_npow<R, T>(), TPL = N / E;
     cx<T> p[B][NP];
     TwChain<T, N, E, Ns * R, Rest...> next;
-    MPC_HD void load(const cx<T> *tw, int tid) {
+    /* tw: the table of an N * ts-point transform */
+    MPC_HD void load(const cx<T> *tw, int tid, int ts = 1) {
         if constexpr (Ns > 1) {
 #pragma unroll
-            for (int b = 0; b < B; ++b) load_powers<R, T>(p[b], tw, ((tid + TPL * b) % Ns) * (N / (Ns * R)));
+            for (int b = 0; b < B; ++b) load_powers<R, T>(p[b], tw, ((tid + TPL * b) % Ns) * (N / (Ns * R)) * ts);
         }
-        next.load(tw, tid);
+        next.load(tw, tid, ts);
     }
 };
 
@@ -359,6 +361,97 @@ template <> struct TPlan<2048> { static constexpr int E = 8; using R = Radices<8
 template <> struct TPlan<1024> { static constexpr int E = 8; using R = Radices<8, 8, 8, 2>; };
 template <> struct TPlan<512>  { static constexpr int E = 8; using R = Radices<8, 8, 8>; };
 template <> struct TPlan<256>  { static constexpr int E = 8; using R = Radices<8, 8, 4>; };
+
+/*
+ * t lines longer than a wavefront's 512 points: NT = R1 * 512.  One radix-R1
+ * step joins the R1 wavefronts of a line; the rest of the transform, a
+ * 512-point one per wavefront, exchanges within the wavefront, which needs no
+ * barrier.  Forward (time to frequency), with n = n' + 512 q, k = k1 + R1 k2:
+ *   X[k1 + R1 k2] = sum_n' W_512^(n' k2) { W_NT^(n' k1) sum_q x[n' + 512 q] W_R1^(q k1) }
+ * the braces are cross_fwd, wavefront k1 then does the n' sum; the inverse
+ * runs backwards.  In time, element m of thread tid is n = tid + TPL m as
+ * everywhere; in frequency it is k = k1 + R1 (lane + 64 m) (t_order), the
+ * order the t-spectral field and its per-frequency tables are kept in.
+ */
+constexpr int t_wave_len(int nt) { return nt < 512 ? nt : 512; }
+/* the frequency index (FFT order) at position pos of a t-spectral line */
+MPC_HD int t_order(int nt, int pos) {
+    const int r1 = nt / t_wave_len(nt);
+    if (r1 == 1) return pos;
+    const int tpl = nt / 8, tid = pos % tpl;
+    return tid / 64 + r1 * (tid % 64 + 64 * (pos / tpl));
+}
+/*
+ * Exchange between the stages of a wavefront's WN-point transform (radix 8,
+ * 8 elements a thread, L = WN / 8 lanes): after the stage at group size Ns,
+ * lane j's output r goes to row r, column j of a pitched array, and each lane
+ * gathers its next elements lane + L m.  Offsets of m and r are constants, so
+ * an exchange takes one base address each way; an array in Stockham order
+ * under an XOR swizzle is as free of bank conflicts but needs an address per
+ * element (100 of 390 instructions of a transform of 8 elements a thread).
+ * The pitches keep the lanes that the LDS serves at once in different banks.
+ * FP32 (8-byte accesses): 16 consecutive lanes over 32 banks, so rows step by
+ * 2 elements after Ns = 1 and by 8 after Ns = 8.  FP64 (16-byte reads): lanes
+ * 0-3, 12-15, 20-23 and 24-27 of each half-wave's 32 (and the complement) over
+ * 64 banks, so rows step by 4 and by 8 (as counted by SQ_LDS_BANK_CONFLICT).
+ */
+template <class T, int WN> struct WaveX {
+    static constexpr int E = 8, L = WN / E;
+    static constexpr int ELEMS = E * (L + 8);            /* of a wavefront's region */
+    template <int Ns> static constexpr int pitch() { return L + (Ns > 1 ? 8 : sizeof(T) == 4 ? 2 : 4); }
+    template <int Ns> static MPC_HD void put(const cx<T> (&v)[E], int lane, cx<T> *lds) {
+#pragma unroll
+        for (int r = 0; r < E; ++r) lds[r * pitch<Ns>() + lane] = v[r];
+    }
+    template <int Ns> static MPC_HD void get(cx<T> (&v)[E], int lane, const cx<T> *lds) {
+        static_assert(Ns == 1 || Ns == 8, "the exchange after a third radix-8 stage is not needed");
+#pragma unroll
+        for (int m = 0; m < E; ++m) {
+            if constexpr (Ns == 1) {
+                v[m] = lds[(lane % 8) * pitch<1>() + lane / 8 + L / 8 * m];
+            } else {
+                constexpr int H = 64 / L;                /* elements m per 64 outputs */
+                v[m] = lds[(lane / 8 + L / 8 * (m % H)) * pitch<8>() + lane % 8 + 8 * (m / H)];
+            }
+        }
+    }
+};
+template <class T, int NT, int R1, int E> struct TCross {
+    static constexpr int WN = WaveX<T, NT / R1>::ELEMS, TPL = NT / E, B = E / R1, NP = tw_npow<R1, T>();
+    cx<T> p[B][NP];                                  /* W_NT^(n' r), n' = tid + TPL b */
+    MPC_HD void load(const cx<T> *tw, int tid) {
+#pragma unroll
+        for (int b = 0; b < B; ++b) load_powers<R1, T>(p[b], tw, tid + TPL * b);
+    }
+    /* lds: the line's R1 regions (WN elements apart), one per wavefront */
+    MPC_HD void fwd(const cx<T> (&v)[E], int tid, cx<T> *lds) const {
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            cx<T> u[R1], w[R1];
+#pragma unroll
+            for (int q = 0; q < R1; ++q) u[q] = v[b + B * q];
+            Dft<R1, -1, T>::run(u);
+            expand_powers<R1, -1>(w, p[b]);
+#pragma unroll
+            for (int r = 0; r < R1; ++r) lds[r * WN + tid + TPL * b] = r ? cmul(u[r], w[r]) : u[r];
+        }
+    }
+    MPC_HD void inv(cx<T> (&v)[E], int tid, const cx<T> *lds) const {
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            cx<T> u[R1], w[R1];
+            expand_powers<R1, +1>(w, p[b]);
+#pragma unroll
+            for (int r = 0; r < R1; ++r) {
+                u[r] = lds[r * WN + tid + TPL * b];
+                if (r) u[r] = cmul(u[r], w[r]);
+            }
+            Dft<R1, +1, T>::run(u);
+#pragma unroll
+            for (int q = 0; q < R1; ++q) v[b + B * q] = u[q];
+        }
+    }
+};
 
 template <int N> struct Plan;
 /* t lines */

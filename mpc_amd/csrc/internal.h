@@ -48,9 +48,9 @@ struct PlasmaK {
 template <class T> struct TArgs {
     cx<T> *field;
     const cx<T> *tw;     /* Nt twiddles exp(-2 pi i k / Nt) */
-    const cx<T> *P;      /* pre table, FFT order, includes 1/Nt; nullptr: already applied */
+    const cx<T> *P;      /* pre table, field's frequency order (t_order), includes 1/Nt; nullptr: already applied */
     const cx<T> *Q;      /* post table (only with out_time) or nullptr */
-    const T *wfft;       /* FFT-order Omega grid */
+    const T *wfft;       /* Omega grid in the field's frequency order */
     double *rho_block;   /* per-block max(ions1 + 2 ions2), may be nullptr */
     PlasmaK pk;
     T dz, gamma, sst_coef; /* sst_coef = gamma2 / w0 */
@@ -154,7 +154,7 @@ struct mpc_ctx_s {
     int snap_pending = 0;
     double guard_tol = -1.0;         /* mpc_set_guard: energy-gain tolerance of mpc_run, < 0 off */
     void *tw_t = nullptr, *tw_x = nullptr;   /* twiddles */
-    void *wfft = nullptr;            /* FFT-order Omega, precision T */
+    void *wfft = nullptr;            /* Omega in the field's frequency order, precision T */
     void *mirror = nullptr;          /* mirror table [y][x] */
     double *rho_block = nullptr;     /* per t-line block */
     int rho_nvalid = 0;              /* entries written by the last plasma t-line launch */

@@ -123,16 +123,17 @@ template int launch_scale<float>(cx<float> *, long, float, hipStream_t);
 /* ---------------------------------------------------------------------- */
 /* SPEC: the field holds the unnormalised t-FFT of each line (the t-spectral
  * state); spec is then read off directly and temp and the line power come
- * from the inverse transform, scaled by 1/nt^2 */
+ * from the inverse transform, scaled by 1/nt^2.  spec leaves in FFT order
+ * (t_order). */
 template <class T, int NT, bool SPEC>
-__global__ void __launch_bounds__(256) k_diag_lines(const cx<T> *f, const cx<T> *tw, long nlines,
+__global__ void __launch_bounds__(TGeo<NT>::THREADS) k_diag_lines(const cx<T> *f, const cx<T> *tw, long nlines,
                                                     double *line_power, double *temp_part, double *spec_part) {
     using G = TGeo<NT>;
     constexpr int E = G::E, TPL = G::TPL, LPB = G::LPB;
     /* with one line per block each thread owns its t values and writes its
      * partial sums itself; with several, the slots are combined in LDS */
     constexpr bool SLOTS = LPB > 1;
-    __shared__ __align__(16) cx<T> lds[LPB * G::FFT_ELEMS];
+    __shared__ __align__(16) cx<T> lds[LPB * TLine<T, G>::ELEMS];
     __shared__ double accT[SLOTS ? NT : 1], accS[SLOTS ? NT : 1];
     __shared__ double lp[LPB][TPL / 64 + 1];
     const int lslot = threadIdx.x / TPL, tid = threadIdx.x % TPL;
@@ -147,6 +148,7 @@ __global__ void __launch_bounds__(256) k_diag_lines(const cx<T> *f, const cx<T> 
     /* a fixed set of line groups per block: deterministic order; the next
      * group's line is loaded while this one is transformed */
     const long ngroups = nlines / LPB;
+    int par = 0;
     cx<T> nxt[E];
     if (blockIdx.x < ngroups) {
         const cx<T> *g0 = f + ((long)blockIdx.x * LPB + lslot) * NT;
@@ -172,7 +174,7 @@ __global__ void __launch_bounds__(256) k_diag_lines(const cx<T> *f, const cx<T> 
         if constexpr (SPEC) {
 #pragma unroll
             for (int m = 0; m < E; ++m) as[m] += (double)v[m].re * v[m].re + (double)v[m].im * v[m].im;
-            line_fft<T, NT, TPlan<NT>, +1, G::PAD>(v, tid, lds + lslot * G::FFT_ELEMS, 1, twi);
+            TLine<T, G>::template run<+1, 0>(v, tid, lds + lslot * TLine<T, G>::ELEMS, par, twi);
             constexpr double inv2 = 1.0 / ((double)NT * (double)NT);
 #pragma unroll
             for (int m = 0; m < E; ++m) {
@@ -187,7 +189,7 @@ __global__ void __launch_bounds__(256) k_diag_lines(const cx<T> *f, const cx<T> 
                 at[m] += p;
                 pw += p;
             }
-            line_fft<T, NT, TPlan<NT>, -1, G::PAD>(v, tid, lds + lslot * G::FFT_ELEMS, 1, twi);
+            TLine<T, G>::template run<-1, 0>(v, tid, lds + lslot * TLine<T, G>::ELEMS, par, twi);
 #pragma unroll
             for (int m = 0; m < E; ++m) as[m] += (double)v[m].re * v[m].re + (double)v[m].im * v[m].im;
         }
@@ -207,7 +209,7 @@ __global__ void __launch_bounds__(256) k_diag_lines(const cx<T> *f, const cx<T> 
 #pragma unroll
         for (int m = 0; m < E; ++m) {
             temp_part[(long)blockIdx.x * NT + tid + TPL * m] = at[m];
-            spec_part[(long)blockIdx.x * NT + tid + TPL * m] = as[m];
+            spec_part[(long)blockIdx.x * NT + t_order(NT, tid + TPL * m)] = as[m];
         }
         return;
     }
@@ -221,7 +223,7 @@ __global__ void __launch_bounds__(256) k_diag_lines(const cx<T> *f, const cx<T> 
     }
     for (int i = threadIdx.x; i < NT; i += blockDim.x) {
         temp_part[(long)blockIdx.x * NT + i] = accT[i];
-        spec_part[(long)blockIdx.x * NT + i] = accS[i];
+        spec_part[(long)blockIdx.x * NT + t_order(NT, i)] = accS[i];
     }
 }
 template <class T, int NT>

@@ -21,9 +21,10 @@ namespace mpc {
  * k_tline<T, G, PLASMA, PERSIST>: a workgroup owns G::LPB t-lines at a time.
  * With PERSIST the grid is what fits on the device at once and each
  * workgroup walks line groups blockIdx.x, + gridDim.x, ...; it loads the
- * twiddle powers and the Omega grid once, and loads the next group's field
- * while it works on the current one, so the HBM latency of a line is hidden
- * behind the previous line's FFTs.  Without PERSIST the grid has one
+ * twiddle powers once and, where registers allow it (TLinePre), the Omega grid
+ * too, and loads the next group's field while it works on the current one, so
+ * the HBM latency of a line is hidden behind the previous line's FFTs.
+ * Without PERSIST the grid has one
  * workgroup per line group and every table is read per line.
  */
 /*
@@ -84,13 +85,31 @@ __device__ __forceinline__ void tline_line(const TArgs<T> &a, cx<T> (&v)[G::E], 
                                      fabs((double)a.dz));
         }
         /* A <- A exp(dz A_nl)  (propagation.c:317-327, complex product) */
+        T mre = (T)0, mim = (T)0;
 #pragma unroll
         for (int m = 0; m < E; ++m) {
-            const T er = exp_t<T>(a.dz * d[m].re);
-            T sn, cs;
-            sincos_t<T>(a.dz * d[m].im, &sn, &cs);
-            const cx<T> z = mk(v[m].re * cs - v[m].im * sn, v[m].re * sn + v[m].im * cs);
-            v[m] = mk(er * z.re, er * z.im);
+            d[m].re *= a.dz;
+            d[m].im *= a.dz;
+            mre = max_abs(mre, d[m].re);
+            mim = max_abs(mim, d[m].im);
+        }
+        if (__all(mre < SmallStep<T>::RE && mim < SmallStep<T>::IM)) {
+#pragma unroll
+            for (int m = 0; m < E; ++m) {
+                T er, sn, cs;
+                small_exp(d[m], er, sn, cs);
+                const cx<T> z = mk(v[m].re * cs - v[m].im * sn, v[m].re * sn + v[m].im * cs);
+                v[m] = mk(er * z.re, er * z.im);
+            }
+        } else {
+#pragma unroll
+            for (int m = 0; m < E; ++m) {
+                const T er = exp_t<T>(d[m].re);
+                T sn, cs;
+                sincos_t<T>(d[m].im, &sn, &cs);
+                const cx<T> z = mk(v[m].re * cs - v[m].im * sn, v[m].re * sn + v[m].im * cs);
+                v[m] = mk(er * z.re, er * z.im);
+            }
         }
         fft(v, Fwd{});
     }
@@ -117,14 +136,20 @@ template <class G> __device__ __forceinline__ void tline_flush_rho(double rmax, 
     __syncthreads();
 }
 
+/* Whether a persistent workgroup loads its next line under the current one's
+ * transforms (and keeps the Omega grid in registers) */
+template <class T, class G, bool PERSIST> constexpr bool TLinePre = PERSIST;
+/* waves per SIMD the kernel is held to */
+template <class T, class G, bool PERSIST>
+constexpr int TLineWaves = sizeof(T) == 8 ? 1 : PERSIST ? 2 : 3;
+
 /* the work of one workgroup: line groups grp, grp + gstride, ... of the
  * field a describes (one group unless PERSIST); its plasma maximum goes to
  * a.rho_block[rho_slot] */
 template <class T, class G, bool PLASMA, bool PERSIST>
 __device__ __forceinline__ void tline_work(const TArgs<T> &a, long grp, long gstride, long rho_slot) {
     using C = TCfg<T, G, PLASMA>;
-    using PL = typename G::PL;
-    using CO = ChainOf<T, G::NT, C::E, typename PL::R>;
+    using LN = TLine<T, G>;
     constexpr int NT = G::NT;
     constexpr int E = C::E, TPL = C::TPL, LPB = C::LPB;
     __shared__ __align__(16) unsigned char smem[LPB * C::LINE_BYTES];
@@ -133,29 +158,32 @@ __device__ __forceinline__ void tline_work(const TArgs<T> &a, long grp, long gst
     if (grp >= ngroups) return;                       /* whole workgroup */
     int tid = tid0, lslot = lslot0;
 
-    std::conditional_t<PERSIST, typename CO::type, NoChain> twc;
+    constexpr bool PRE = TLinePre<T, G, PERSIST>;
+    std::conditional_t<PERSIST, typename LN::Chain, NoChain> twc;
     T wk[E];
     if constexpr (PERSIST) {
         twc.load(a.tw, tid);
-        if (a.do_nl && a.sst_on) {
+        if (PRE && a.do_nl && a.sst_on) {
 #pragma unroll
             for (int m = 0; m < E; ++m) wk[m] = gload(a.wfft, tid + TPL * m);
         }
     }
     unsigned char *lraw;
     cx<T> *L;
+    int par = 0;                                      /* the exchange buffer the next transform uses */
     auto fft = [&](cx<T>(&x)[E], auto dir) {
         constexpr int DIR = decltype(dir)::value;
-        if constexpr (PERSIST) CO::template fft<DIR, G::PAD, C::BOFF>(x, tid, L, 1, twc);
-        else line_fft<T, NT, PL, DIR, G::PAD, C::BOFF>(x, tid, L, 1, a.tw);
+        if constexpr (PERSIST) LN::template run<DIR, C::BOFF>(x, tid, L, par, twc);
+        else LN::template run<DIR, C::BOFF>(x, tid, L, par, a.tw);
     };
 
     cx<T> nxt[E];
-    {
-        const cx<T> *g0 = a.field + (grp * LPB + lslot) * NT;
+    auto load = [&](long g) {
+        const cx<T> *p = a.field + (g * LPB + lslot) * NT;
 #pragma unroll
-        for (int m = 0; m < E; ++m) nxt[m] = gload(g0, tid + TPL * m);
-    }
+        for (int m = 0; m < E; ++m) nxt[m] = gload(p, tid + TPL * m);
+    };
+    if constexpr (PRE) load(grp);
     double rmax = 0.0;
     for (;;) {
         /* tid and lslot re-enter as opaque values each iteration, so the
@@ -164,21 +192,18 @@ __device__ __forceinline__ void tline_work(const TArgs<T> &a, long grp, long gst
         tid = tid0;
         lslot = lslot0;
         asm volatile("" : "+v"(tid), "+v"(lslot));
-        if constexpr (PERSIST) opaque_chain(twc);
+        if constexpr (PERSIST) opaque_line(twc);
         lraw = smem + lslot * C::LINE_BYTES;
         L = reinterpret_cast<cx<T> *>(lraw);
         cx<T> *g = a.field + (grp * LPB + lslot) * NT;
+        if constexpr (!PRE) load(grp);
         cx<T> v[E];
 #pragma unroll
         for (int m = 0; m < E; ++m) v[m] = nxt[m];
         const long gnext = grp + gstride;
-        tline_line<T, G, PLASMA, PERSIST>(a, v, tid, lraw, wk, rmax, fft, [&] {
-            if constexpr (PERSIST) {
-                if (gnext < ngroups) {
-                    const cx<T> *gn = a.field + (gnext * LPB + lslot) * NT;
-#pragma unroll
-                    for (int m = 0; m < E; ++m) nxt[m] = gload(gn, tid + TPL * m);
-                }
+        tline_line<T, G, PLASMA, PRE>(a, v, tid, lraw, wk, rmax, fft, [&] {
+            if constexpr (PRE) {
+                if (gnext < ngroups) load(gnext);
             }
         });
 #pragma unroll
@@ -191,13 +216,11 @@ __device__ __forceinline__ void tline_work(const TArgs<T> &a, long grp, long gst
     }
 }
 
-/* FP32: the persistent form is held to two waves per SIMD (256 VGPRs) and
- * the per-group form to three (168 VGPRs, which its plasma LDS allows too).
- * The persistent form fits; the per-group form spills (tens of VGPRs at 1024
- * and 2048 points, since it loads every stage twiddle), and the tuner keeps
- * whichever is faster */
+/* FP32: the persistent form is held to two waves per SIMD (256 VGPRs), the
+ * per-group form to three (168), which its plasma LDS allows too.  The tuner
+ * keeps whichever is faster */
 template <class T, class G, bool PLASMA, bool PERSIST>
-__global__ void __launch_bounds__((TCfg<T, G, PLASMA>::THREADS), sizeof(T) == 4 ? (PERSIST ? 2 : 3) : 1)
+__global__ void __launch_bounds__((TCfg<T, G, PLASMA>::THREADS), (TLineWaves<T, G, PERSIST>))
 k_tline(TArgs<T> a) {
     tline_work<T, G, PLASMA, PERSIST>(a, blockIdx.x, gridDim.x, blockIdx.x);
 }
@@ -232,15 +255,14 @@ k_tline_batch(const TArgs<T> *__restrict__ d, const long *__restrict__ gstart, i
  * field's arguments, twiddle powers and Omega grid, and flushes its plasma
  * maximum for the field it leaves to slot j = its first group in that field,
  * so the slots [0, min(grid, groups)) of each field are written exactly
- * once.  The next group is prefetched across field boundaries too.  The
- * per-line arithmetic is the persistent per-field kernel's (tline_line).
+ * once.  Where the per-field form loads ahead this one does too, across field
+ * boundaries.  The per-line arithmetic is the persistent per-field kernel's (tline_line).
  */
 template <class T, class G, bool PLASMA>
 __device__ __forceinline__ void tline_work_batch(const TArgs<T> *__restrict__ d, const long *__restrict__ gstart,
                                                  int n) {
     using C = TCfg<T, G, PLASMA>;
-    using PL = typename G::PL;
-    using CO = ChainOf<T, G::NT, C::E, typename PL::R>;
+    using LN = TLine<T, G>;
     constexpr int NT = G::NT;
     constexpr int E = C::E, TPL = C::TPL, LPB = C::LPB;
     __shared__ __align__(16) unsigned char smem[LPB * C::LINE_BYTES];
@@ -261,11 +283,12 @@ __device__ __forceinline__ void tline_work_batch(const TArgs<T> *__restrict__ d,
     long first = g - gstart[p];
     int tid = tid0, lslot = lslot0;
 
-    typename CO::type twc;
+    constexpr bool PRE = TLinePre<T, G, true>;
+    typename LN::Chain twc;
     T wk[E];
     auto load_field = [&] {
         twc.load(a.tw, tid);
-        if (a.do_nl && a.sst_on) {
+        if (PRE && a.do_nl && a.sst_on) {
 #pragma unroll
             for (int m = 0; m < E; ++m) wk[m] = gload(a.wfft, tid + TPL * m);
         }
@@ -273,38 +296,38 @@ __device__ __forceinline__ void tline_work_batch(const TArgs<T> *__restrict__ d,
     load_field();
     unsigned char *lraw;
     cx<T> *L;
+    int par = 0;                                      /* the exchange buffer the next transform uses */
     auto fft = [&](cx<T>(&x)[E], auto dir) {
         constexpr int DIR = decltype(dir)::value;
-        CO::template fft<DIR, G::PAD, C::BOFF>(x, tid, L, 1, twc);
+        LN::template run<DIR, C::BOFF>(x, tid, L, par, twc);
     };
 
     cx<T> nxt[E];
-    {
-        const cx<T> *g0 = a.field + ((g - gstart[p]) * LPB + lslot) * NT;
+    auto load = [&](const cx<T> *f, long gl) {
+        const cx<T> *src = f + (gl * LPB + lslot) * NT;
 #pragma unroll
-        for (int m = 0; m < E; ++m) nxt[m] = gload(g0, tid + TPL * m);
-    }
+        for (int m = 0; m < E; ++m) nxt[m] = gload(src, tid + TPL * m);
+    };
+    if constexpr (PRE) load(a.field, g - gstart[p]);
     double rmax = 0.0;
     for (;;) {
         tid = tid0;
         lslot = lslot0;
         asm volatile("" : "+v"(tid), "+v"(lslot));
-        opaque_chain(twc);
+        opaque_line(twc);
         lraw = smem + lslot * C::LINE_BYTES;
         L = reinterpret_cast<cx<T> *>(lraw);
         cx<T> *gp = a.field + ((g - gstart[p]) * LPB + lslot) * NT;
+        if constexpr (!PRE) load(a.field, g - gstart[p]);
         cx<T> v[E];
 #pragma unroll
         for (int m = 0; m < E; ++m) v[m] = nxt[m];
         const long gn = g + gridDim.x;
         int pn = p;
         while (pn + 1 < n && gstart[pn + 1] <= gn) ++pn;
-        tline_line<T, G, PLASMA, true>(a, v, tid, lraw, wk, rmax, fft, [&] {
-            if (gn < total) {
-                const cx<T> *fn = pn == p ? a.field : d[pn].field;
-                const cx<T> *src = fn + ((gn - gstart[pn]) * LPB + lslot) * NT;
-#pragma unroll
-                for (int m = 0; m < E; ++m) nxt[m] = gload(src, tid + TPL * m);
+        tline_line<T, G, PLASMA, PRE>(a, v, tid, lraw, wk, rmax, fft, [&] {
+            if constexpr (PRE) {
+                if (gn < total) load(pn == p ? a.field : d[pn].field, gn - gstart[pn]);
             }
         });
 #pragma unroll
@@ -326,7 +349,7 @@ __device__ __forceinline__ void tline_work_batch(const TArgs<T> *__restrict__ d,
 }
 
 template <class T, class G, bool PLASMA>
-__global__ void __launch_bounds__((TCfg<T, G, PLASMA>::THREADS), sizeof(T) == 4 ? 2 : 1)
+__global__ void __launch_bounds__((TCfg<T, G, PLASMA>::THREADS), (TLineWaves<T, G, true>))
 k_tline_batch_p(const TArgs<T> *__restrict__ d, const long *__restrict__ gstart, int n) {
     tline_work_batch<T, G, PLASMA>(d, gstart, n);
 }
