@@ -136,12 +136,18 @@ template <class G> __device__ __forceinline__ void tline_flush_rho(double rmax, 
     __syncthreads();
 }
 
-/* Whether a persistent workgroup loads its next line under the current one's
- * transforms (and keeps the Omega grid in registers) */
-template <class T, class G, bool PERSIST> constexpr bool TLinePre = PERSIST;
+/*
+ * Whether a persistent workgroup loads its next line under the current one's
+ * transforms (and keeps the Omega grid in registers).  In FP32 those 24
+ * registers are worth more as a third wave per SIMD, whose work covers the
+ * loads: 256x256x2048 1.10 -> 1.03 ms, 128x128x512 60 -> 56 us.  A 4096-point
+ * line's workgroup of eight waves leaves room for two per SIMD only (160
+ * against 175 us at 64x64x4096), and FP64 for one.
+ */
+template <class T, class G, bool PERSIST> constexpr bool TLinePre = PERSIST && (sizeof(T) == 8 || G::NT == 4096);
 /* waves per SIMD the kernel is held to */
 template <class T, class G, bool PERSIST>
-constexpr int TLineWaves = sizeof(T) == 8 ? 1 : PERSIST ? 2 : 3;
+constexpr int TLineWaves = sizeof(T) == 8 ? 1 : TLinePre<T, G, PERSIST> ? 2 : 3;
 
 /* the work of one workgroup: line groups grp, grp + gstride, ... of the
  * field a describes (one group unless PERSIST); its plasma maximum goes to
@@ -216,8 +222,8 @@ __device__ __forceinline__ void tline_work(const TArgs<T> &a, long grp, long gst
     }
 }
 
-/* FP32: the persistent form is held to two waves per SIMD (256 VGPRs), the
- * per-group form to three (168), which its plasma LDS allows too.  The tuner
+/* FP32: both forms are held to three waves per SIMD (168 VGPRs; two where the
+ * persistent form loads ahead), which their plasma LDS allows too.  The tuner
  * keeps whichever is faster */
 template <class T, class G, bool PLASMA, bool PERSIST>
 __global__ void __launch_bounds__((TCfg<T, G, PLASMA>::THREADS), (TLineWaves<T, G, PERSIST>))
