@@ -1115,38 +1115,42 @@ template <class T> static int two_steps_f(mpc_ctx *c, double dzz, double z, int 
     return rc;
 }
 
-/* a t-spectral field (left so by mpc_run or mpc_run_adaptive) back to the
- * time domain, in place: the 1/nt of the transform pair, then the inverse
- * transform.  Always with the per-group t-line form, whatever variant the
- * context is tuned to (in FP64 the forms' twiddle products round
+/* c's t-spectral field (left so by mpc_run or mpc_run_adaptive) in time, to
+ * out (which may be the field) or to planes: the 1/nt of the transform pair,
+ * then the inverse transform.  Always by k_tline_view, whatever variant the
+ * context is tuned to (in FP64 the t-line forms' twiddle products round
  * differently), so the time-domain field does not depend on the tuning. */
-template <class T> static int to_time(mpc_ctx *c) {
-    if (!c->domain_freq) return 0;
+template <class T> static int view_t(mpc_ctx *c, void *out, float *planes, double scale) {
     const cx<T> *Q0 = get_table<T>(c, 't', 0.0);
     if (!Q0) return MPC_ENOMEM;
-    const int keep = c->tvar;
-    c->tvar = 1;
-    const int rc = sweep_t<T>(c, nullptr, Q0, true, false, true, 0.0);
-    c->tvar = keep;
-    RCHK(rc);
+    tic(c, 0);
+    const int rc = launch_tline_view<T>((const cx<T> *)c->field, Q0, (const cx<T> *)c->tw_t, c->nxy, c->nt, (cx<T> *)out,
+                                        planes, scale, c->stream);
+    toc(c, 0);
+    return rc;
+}
+static int view(mpc_ctx *c, void *out, float *planes, double scale) {
+    return c->prec == MPC_F32 ? view_t<float>(c, out, planes, scale) : view_t<double>(c, out, planes, scale);
+}
+/* the field back to the time domain, in place */
+static int to_time_any(mpc_ctx *c) {
+    if (!c->domain_freq) return 0;
+    RCHK(view(c, c->field, nullptr, 1.0));
     c->domain_freq = 0;
     return 0;
 }
-static int to_time_any(mpc_ctx *c) { return c->prec == MPC_F32 ? to_time<float>(c) : to_time<double>(c); }
-/* fn on a time-domain view of c's field that leaves c as it was (a read: a
- * t-spectral field is copied to aux1 and transformed there), so reading the
- * field never changes the path a later run takes */
+/* fn on a time-domain view of c's field that leaves c as it was (a
+ * t-spectral field is transformed into aux1), so reading the field never
+ * changes the path a later run takes */
 template <class F> static int time_view(mpc_ctx *c, F &&fn) {
     if (!c->domain_freq) return fn();
     const size_t bytes = c->esz * (size_t)c->N;
     if (!c->aux1 && hipMalloc(&c->aux1, bytes) != hipSuccess) return MPC_ENOMEM;
-    HIPCHK(hipMemcpyAsync(c->aux1, c->field, bytes, hipMemcpyDeviceToDevice, c->stream));
+    RCHK(view(c, c->aux1, nullptr, 1.0));
     void *keep = c->field;
     c->field = c->aux1;
-    int rc = to_time_any(c);
-    if (!rc) rc = fn();
+    const int rc = fn();
     c->field = keep;
-    c->domain_freq = 1;
     return rc;
 }
 
@@ -1293,10 +1297,10 @@ extern "C" int mpc_snapshot_wait(mpc_ctx *c, const cufftDoubleComplex **A) {
 extern "C" int mpc_export_planar(mpc_ctx *c, float *planes, double scale) {
     if (!c || !planes) return MPC_EINVAL;
     const double s = scale * c->ascale;
-    const int rc = time_view(c, [&] {
-        return c->prec == MPC_F32 ? launch_planar<float>((cx<float> *)c->field, planes, c->N, s, 1, c->stream)
-                                  : launch_planar<double>((cx<double> *)c->field, planes, c->N, s, 1, c->stream);
-    });
+    const int rc = c->domain_freq
+        ? view(c, nullptr, planes, s)
+        : (c->prec == MPC_F32 ? launch_planar<float>((cx<float> *)c->field, planes, c->N, s, 1, c->stream)
+                              : launch_planar<double>((cx<double> *)c->field, planes, c->N, s, 1, c->stream));
     return finish(c, rc);
 }
 extern "C" int mpc_import_planar(mpc_ctx *c, const float *planes, double scale) {

@@ -78,6 +78,11 @@ template <class T> struct AArgs {
  * entries the launch writes */
 template <class T> int launch_tline(const TArgs<T> &a, int nt, bool plasma, int variant, hipStream_t s, int *nblocks);
 template <class T> int launch_axis(const AArgs<T> &a, int n, int outer, int variant, hipStream_t s);
+/* the time-domain form of a t-spectral field: to out (which may be field), or (planes != nullptr) times scale to two
+ * float planes */
+template <class T>
+int launch_tline_view(const cx<T> *field, const cx<T> *Q, const cx<T> *tw, long nlines, int nt, cx<T> *out,
+                      float *planes, double scale, hipStream_t s);
 int tline_variants(void);
 int axis_variants(void);
 template <class T> int launch_to_internal(const double *src, cx<T> *dst, int nx, int ny, int nt, double scale,
