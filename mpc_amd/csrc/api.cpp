@@ -207,7 +207,6 @@ extern "C" int mpc_create(const mpc_params *p, int precision, mpc_ctx **out) {
         c->diag_nblocks = (int)std::max(1L, std::min(1024L, dgroups));
         if (hipMalloc((void **)&c->diag_part, sizeof(double) * 2 * (size_t)c->diag_nblocks * c->nt) != hipSuccess ||
             hipMalloc((void **)&c->diag_line, sizeof(double) * (size_t)c->nxy) != hipSuccess ||
-            hipMalloc((void **)&c->diag_out, sizeof(double) * 2 * (size_t)c->nt) != hipSuccess ||
             hipMalloc((void **)&c->err_part, sizeof(double) * 2 * 1024) != hipSuccess)
             rc = MPC_ENOMEM;
     }
@@ -229,9 +228,10 @@ extern "C" void mpc_destroy(mpc_ctx *c) {
     if (c->snap_ready) (void)hipEventDestroy(c->snap_ready);
     if (c->snap_done) (void)hipEventDestroy(c->snap_done);
     if (c->pinned) (void)hipHostFree(c->pinned);
+    if (c->diag_host) (void)hipHostFree(c->diag_host);
     free_tables(c);
     void *bufs[] = {c->field, c->aux1, c->aux2, c->staging, c->tw_t, c->tw_x, c->wfft, c->mirror,
-                    c->rho_block, c->diag_part, c->diag_line, c->diag_out, c->err_part, c->rich_err, c->rich_lp};
+                    c->rho_block, c->diag_part, c->diag_line, c->err_part, c->rich_err, c->rich_lp};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     for (auto &e : c->evs) {
@@ -1329,8 +1329,39 @@ extern "C" int mpc_calibrate(mpc_ctx *c) {
 /* ------------------------------------------------------------------------ */
 /* diagnostics                                                               */
 /* ------------------------------------------------------------------------ */
+/* the pinned buffer kernels leave host-side results in */
+static int diag_host(mpc_ctx *c) {
+    if (c->diag_host) return 0;
+    const size_t n = 2 * (size_t)c->nt + (size_t)c->nxy + 1;
+    if (hipHostMalloc((void **)&c->diag_host, sizeof(double) * n, hipHostMallocDefault) != hipSuccess) {
+        c->diag_host = nullptr;
+        return MPC_ENOMEM;
+    }
+    return 0;
+}
+/* BP1[x] = sum_{y,t}, BP2[y] = sum_{x,t} (propagation.c:343-354) of the line
+ * powers times scale, either may be nullptr.  Every sum adds its lines in
+ * index order; four rows go together, so that their chains overlap. */
+static void line_profiles(const mpc_ctx *c, const double *lp, double scale, double *BP1, double *BP2) {
+    if (BP1) std::fill(BP1, BP1 + c->nx, 0.0);
+    for (int j = 0; j < c->ny; j += 4) {             /* transverse sizes are multiples of 16 */
+        double s[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int i = 0; i < c->nx; i++) {
+            double b = BP1 ? BP1[i] : 0.0;
+            for (int r = 0; r < 4; r++) {
+                const double v = lp[(size_t)(j + r) * c->nx + i] * scale;
+                s[r] += v;
+                b += v;
+            }
+            if (BP1) BP1[i] = b;
+        }
+        if (BP2) std::copy(s, s + 4, BP2 + j);
+    }
+}
+
 extern "C" int mpc_diagnostics(mpc_ctx *c, mpc_diag *d) {
     if (!c || !d) return MPC_EINVAL;
+    RCHK(diag_host(c));
     /* either domain: a t-spectral field gives spec directly and temp and the
      * line powers through the inverse transform */
     const int nb = c->diag_nblocks;
@@ -1340,15 +1371,12 @@ extern "C" int mpc_diagnostics(mpc_ctx *c, mpc_diag *d) {
         ? launch_diag_lines<float>((const cx<float> *)c->field, (const cx<float> *)c->tw_t, c->nt, c->nxy, c->diag_line, tp, sp, nb, spec, c->stream)
         : launch_diag_lines<double>((const cx<double> *)c->field, (const cx<double> *)c->tw_t, c->nt, c->nxy, c->diag_line, tp, sp, nb, spec, c->stream);
     RCHK(rc);
-    RCHK(launch_reduce_cols(tp, nb, c->nt, c->diag_out, c->stream));
-    RCHK(launch_reduce_cols(sp, nb, c->nt, c->diag_out + c->nt, c->stream));
-    std::vector<double> ts(2 * (size_t)c->nt), lp((size_t)c->nxy), rb;
-    HIPCHK(hipMemcpyAsync(ts.data(), c->diag_out, sizeof(double) * 2 * c->nt, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipMemcpyAsync(lp.data(), c->diag_line, sizeof(double) * c->nxy, hipMemcpyDeviceToHost, c->stream));
+    const long nrho = c->p.plasm == 1 ? std::min<long>(c->rho_nvalid, c->rho_nblocks) : 0;
+    RCHK(launch_diag_finish(tp, nb, c->nt, c->diag_line, c->nxy, c->rho_block, nrho, c->diag_host, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     const double sc2 = c->ascale * c->ascale;
+    std::vector<double> ts(c->diag_host, c->diag_host + 2 * c->nt);
     for (double &v : ts) v *= sc2;
-    for (double &v : lp) v *= sc2;
     double e = 0.0;
     for (int k = 0; k < c->nt; k++) e += ts[k];
     d->energy_sum = e;
@@ -1361,24 +1389,8 @@ extern "C" int mpc_diagnostics(mpc_ctx *c, mpc_diag *d) {
         s0 += sv; s1 += om * sv; s2 += om * om * sv;
     }
     d->spec_rms_width = s0 > 0 ? std::sqrt(std::max(0.0, s2 / s0 - (s1 / s0) * (s1 / s0))) : 0.0;
-    /* BP1[x] = sum_{y,t}, BP2[y] = sum_{x,t} (propagation.c:343-354) */
-    /* BP1 row by row (each BP1[i] still adds its lines in j order, as a
-     * column walk would, with contiguous reads) */
-    if (d->BP1) {
-        std::fill(d->BP1, d->BP1 + c->nx, 0.0);
-        for (int j = 0; j < c->ny; j++)
-            for (int i = 0; i < c->nx; i++) d->BP1[i] += lp[(size_t)j * c->nx + i];
-    }
-    if (d->BP2) for (int j = 0; j < c->ny; j++) { double s = 0; for (int i = 0; i < c->nx; i++) s += lp[(size_t)j * c->nx + i]; d->BP2[j] = s; }
-    d->rho_peak = 0.0;
-    if (c->p.plasm == 1) {
-        rb.resize((size_t)std::min<long>(c->rho_nvalid, c->rho_nblocks));
-        if (!rb.empty())
-            HIPCHK(hipMemcpy(rb.data(), c->rho_block, sizeof(double) * rb.size(), hipMemcpyDeviceToHost));
-        double mx = 0.0;
-        for (double v : rb) mx = std::max(mx, v);
-        d->rho_peak = mx * c->p.rho_nt;
-    }
+    line_profiles(c, c->diag_host + 2 * c->nt, sc2, d->BP1, d->BP2);
+    d->rho_peak = c->p.plasm == 1 ? c->diag_host[2 * c->nt + c->nxy] * c->p.rho_nt : 0.0;
     return 0;
 }
 
@@ -1423,13 +1435,15 @@ template <class T> static int adaptive(mpc_ctx *c, double *z, double *dzz, int *
     if (!c->aux2 && hipMalloc(&c->aux2, bytes) != hipSuccess) return MPC_ENOMEM;
     const long ntiles = axis_richardson_tiles(c->prec, c->nt, c->nx);
     const long nchunks = ntiles / c->nx;
-    if (!c->rich_err && hipMalloc((void **)&c->rich_err, sizeof(double) * (2 * (size_t)ntiles + 2)) != hipSuccess)
+    if (!c->rich_err && hipMalloc((void **)&c->rich_err, sizeof(double) * 2 * (size_t)ntiles) != hipSuccess)
         return MPC_ENOMEM;
     if (!c->rich_lp && hipMalloc((void **)&c->rich_lp, sizeof(double) * (size_t)nchunks * c->nxy) != hipSuccess)
         return MPC_ENOMEM;
     int acc = 0, guard = 0;
-    std::vector<double> BP1(c->nx), BP2(c->ny), lp((size_t)c->nxy);
-    double y1[4] = {0, 0, 0, 0}, y2[4] = {0, 0, 0, 0}, bps = 0, norms[2];
+    RCHK(diag_host(c));
+    std::vector<double> BP1(c->nx), BP2(c->ny);
+    double y1[4] = {0, 0, 0, 0}, y2[4] = {0, 0, 0, 0}, bps = 0;
+    const double *norms = c->diag_host;                  /* two, then the line powers */
     RichOut ro;
     ro.err_part = c->rich_err;
     ro.lp_part = c->rich_lp;
@@ -1456,17 +1470,12 @@ template <class T> static int adaptive(mpc_ctx *c, double *z, double *dzz, int *
         if (!rc) rc = two_steps_f<T>(c, dz, *z, signmem, A, &ro);   /* sub-steps at z and z + dz */
         c->field = A;
         RCHK(rc);
-        RCHK(launch_sum_pairs(c->rich_err, ntiles, c->rich_err + 2 * ntiles, c->stream));
-        RCHK(launch_reduce_cols(c->rich_lp, (int)nchunks, (int)c->nxy, c->diag_line, c->stream));
-        HIPCHK(hipMemcpyAsync(norms, c->rich_err + 2 * ntiles, sizeof norms, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipMemcpyAsync(lp.data(), c->diag_line, sizeof(double) * c->nxy, hipMemcpyDeviceToHost, c->stream));
+        RCHK(launch_sum_pairs(c->rich_err, ntiles, c->diag_host, c->stream));
+        RCHK(launch_reduce_cols(c->rich_lp, (int)nchunks, (int)c->nxy, c->diag_host + 2, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
         if (c->timing) resolve_timing(c);
         /* BP and calc1oes of C2 for the step-size cap (propagation.c:343-362) */
-        std::fill(BP1.begin(), BP1.end(), 0.0);          /* row by row; each BP1[i] adds in j order */
-        for (int j = 0; j < c->ny; j++)
-            for (int i = 0; i < c->nx; i++) BP1[i] += lp[(size_t)j * c->nx + i];
-        for (int j = 0; j < c->ny; j++) { double sm = 0; for (int i = 0; i < c->nx; i++) sm += lp[(size_t)j * c->nx + i]; BP2[j] = sm; }
+        line_profiles(c, c->diag_host + 2, 1.0, BP1.data(), BP2.data());
         int dims[3] = {c->nx, c->ny, c->nt};
         calc1oes(BP1.data(), dims, c->r.data(), &bps, y1);
         calc1oes(BP2.data(), dims, c->r.data(), &bps, y2);

@@ -96,6 +96,8 @@ template <class T> int launch_diag_lines(const cx<T> *f, const cx<T> *tw, int nt
                                          double *line_power, double *temp_part, double *spec_part,
                                          int nblocks, bool spectral, hipStream_t s);
 int launch_reduce_cols(const double *part, int nrows, int ncols, double *out, hipStream_t s);
+int launch_diag_finish(const double *part, int nrows, int nt, const double *lines, long nlines, const double *rho,
+                       long nrho, double *host, hipStream_t s);
 template <class T> int launch_err_partials(const cx<T> *c1, const cx<T> *c2, long n, double *part,
                                            int nblocks, hipStream_t s);
 /* the last y sweep of an adaptive fine branch fused with the error norms,
@@ -166,9 +168,9 @@ struct mpc_ctx_s {
     long rho_nblocks = 0;
     double *diag_part = nullptr;     /* diagnostics partials */
     double *diag_line = nullptr;     /* per-line power */
-    double *diag_out = nullptr;      /* reduced temp/spec */
+    double *diag_host = nullptr;     /* pinned, 2 nt + nxy + 1: what diagnostics and adaptive attempts bring back */
     double *err_part = nullptr;
-    double *rich_err = nullptr;      /* adaptive: per-tile error norms of the fused sweep, then their sums */
+    double *rich_err = nullptr;      /* adaptive: per-tile error norms of the fused sweep */
     double *rich_lp = nullptr;       /* adaptive: per-chunk line powers of C2 */
     int diag_nblocks = 0;
     mpc::PlasmaK pk{};

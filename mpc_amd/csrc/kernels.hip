@@ -280,6 +280,68 @@ int launch_reduce_cols(const double *part, int nrows, int ncols, double *out, hi
     return hipGetLastError() == hipSuccess ? 0 : MPC_EHIP;
 }
 
+/*
+ * The last kernel of the diagnostics: host (pinned host memory, written over
+ * the bus) receives the 2 nt column sums of part (temp and spec), then the nlines line
+ * powers, then the largest of the nrho plasma maxima (0 for none; a NaN is
+ * passed over).  The first blocks sum DF_COLS columns each, DF_PARTS threads
+ * per column over rows q, q + DF_PARTS, ..., then in a fixed order; the next
+ * copy the line powers; the last takes the maximum.  Written this way the
+ * results need no copies: two column sums of 8 blocks each and three copies to
+ * pageable memory were 44 us of kernels and three waits (64x64x512, FP64), now
+ * 4 us and one.
+ */
+constexpr int DF_COLS = 16, DF_PARTS = 64, DF_THREADS = DF_COLS * DF_PARTS;
+__global__ void __launch_bounds__(DF_THREADS) k_diag_finish(const double *__restrict__ part, int nrows, int nt,
+                                                            const double *__restrict__ lines, long nlines,
+                                                            const double *__restrict__ rho, long nrho,
+                                                            double *__restrict__ host) {
+    __shared__ double ps[DF_THREADS / 64][DF_COLS];
+    const int tid = threadIdx.x;
+    const int ncols = 2 * nt, cblocks = ncols / DF_COLS;
+    if ((int)blockIdx.x < cblocks) {
+        const int cl = tid % DF_COLS, q = tid / DF_COLS;
+        const int c = blockIdx.x * DF_COLS + cl;
+        const double *p = part + (c < nt ? c : (long)nrows * nt + c - nt);
+        double s = 0.0;
+#pragma unroll 4
+        for (int r = q; r < nrows; r += DF_PARTS) s += p[(long)r * nt];
+        s += __shfl_xor(s, 16);
+        s += __shfl_xor(s, 32);
+        if (tid % 64 < DF_COLS) ps[tid / 64][cl] = s;
+        __syncthreads();
+        if (tid < DF_COLS) {
+            double t = 0.0;
+#pragma unroll
+            for (int k = 0; k < DF_THREADS / 64; ++k) t += ps[k][tid];
+            host[c] = t;
+        }
+    } else if (blockIdx.x + 1 < gridDim.x) {
+        const long i = (long)(blockIdx.x - cblocks) * DF_THREADS + tid;
+        if (i < nlines) host[ncols + i] = lines[i];
+    } else {
+        double r = 0.0;
+        for (long i = tid; i < nrho; i += DF_THREADS) r = fmax(r, rho[i]);
+        for (int o = 32; o > 0; o >>= 1) r = fmax(r, __shfl_down(r, o));
+        if (tid % 64 == 0) ps[tid / 64][0] = r;
+        __syncthreads();
+        if (tid == 0) {
+#pragma unroll
+            for (int k = 1; k < DF_THREADS / 64; ++k) r = fmax(r, ps[k][0]);
+            host[ncols + nlines] = r;
+        }
+    }
+}
+/* part: temp [nrows][nt], then spec [nrows][nt]; host: 2 nt + nlines + 1 values */
+int launch_diag_finish(const double *part, int nrows, int nt, const double *lines, long nlines, const double *rho,
+                       long nrho, double *host, hipStream_t s) {
+    if (nrows <= 0 || nt <= 0 || nt % DF_COLS || nlines <= 0) return MPC_EINVAL;
+    const long nb = 2 * nt / DF_COLS + (nlines + DF_THREADS - 1) / DF_THREADS + 1;
+    hipLaunchKernelGGL(k_diag_finish, dim3((unsigned)nb), dim3(DF_THREADS), 0, s, part, nrows, nt, lines, nlines, rho,
+                       nrho, host);
+    return hipGetLastError() == hipSuccess ? 0 : MPC_EHIP;
+}
+
 /* ---------------------------------------------------------------------- */
 /* setStep's error norms (propagation.c:625-631), fixed-order sums, energy  */
 /*                                                                         */
