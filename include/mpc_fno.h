@@ -105,15 +105,19 @@ int mpc_fno_mix_bwd(const float *V, const float *dU, const float *Rr, const floa
  *   y == NULL:   C1 = v' Ft, the next layer's t-DFT;
  *   otherwise    (no act) the head: y[b][0..2] = q2w GELU(q1w v' + q1) + q2 +
  *                x[b][0..2], h hidden channels, x with batch stride x_bs.
- * Gt (n2 x nt) and Ft (nt x n2) are given packed (mpc_fno_pack, which rounds
- * them to BF16); V6 and v' are rounded to BF16 as operands of
- * the t-DFTs, as mpc_gemm_bf16 does; the channel maps are FP32.  Supported
- * where mpc_fno_column_fits says so (width 8, 16, 32 or 64, cin 4, nt <= 256,
- * even n2 <= 64, h a
- * power of two <= 64); otherwise MPC_EUNSUPP.
+ *   bwd = 1 (training's backward between two layers): v is the layer's dz, w
+ *                its channel map transposed, V6 its transposed mode path's
+ *                result, Gt = Ft^T and Ft = Gt^T; no bias.  With zin, the
+ *                pre-activations of the layer below: out = (V6 Gt + w v)
+ *                GELU'(zin) and C1 = out Ft; without, out = V6 Gt + w v.
+ * out may be v.  Gt (n2 x nt) and Ft (nt x n2) are given packed (mpc_fno_pack,
+ * which rounds them to BF16); V6 and v' are rounded to BF16 as operands of the
+ * t-DFTs, as mpc_gemm_bf16 does; the channel maps are FP32.  Supported where
+ * mpc_fno_column_fits says so (width 8, 16, 32 or 64, cin 4, nt <= 256, even
+ * n2 <= 64, h a power of two <= 64); otherwise MPC_EUNSUPP.
  */
 typedef struct {
-    int nb, width, npos, nt, n2, act, h, pad_;
+    int nb, width, npos, nt, n2, act, h, bwd;
     const float *v;
     long v_bs;
     const float *V6;
@@ -123,6 +127,7 @@ typedef struct {
     const float *q1w, *q1, *q2w, *q2, *x;
     long x_bs;
     float *y;
+    const float *zin;
 } mpc_fno_col;
 
 int mpc_fno_column(const mpc_fno_col *a, void *stream);

@@ -49,7 +49,13 @@ __device__ __forceinline__ int drow(int r, int h) { return 8 * (r / 4) + 4 * h +
  *   KIND 1, layer: z = V6 Gt + Wm v + bias; v' = GELU(z) if act; ZS (training):
  *           z is stored too and the GELU is the training path's
  *   KIND 2, last:  as KIND 1, then y = Q2 GELU(Q1 v' + q1) + q2 + x[:, :2]
- * Kinds 0 and 1 then form C1 = v' Ft, from v' rounded to BF16 in LDS.
+ *   KIND 3, backward: dz' = (V6 Gt + Wm dz) GELU'(zin), with V6 the transposed
+ *           mode path's result, Gt = Ft^T and Wm the transposed channel map of
+ *           the layer above, zin this layer's pre-activation
+ *   KIND 4, backward through the first layer: V6 Gt + Wm dz only
+ * Kinds 0, 1 and 3 then form C1 = v' Ft (3: Ft = Gt^T), from v' rounded to BF16
+ * in LDS.  Kind 3 at batch 4 of 64 x 64 x 256 points, width 32, moves 3 streams
+ * of 0.54 GB in 395 us; the four kernels it stands for took 1100.
  * LDS at W = 32, T = 256: Ft 33 KB, v' 17 KB, V6 5 KB, Wm 4 KB: two workgroups
  * (four waves per SIMD) fit on a CU, so one's loads and stores run under the
  * other's products and GELUs.
@@ -74,6 +80,7 @@ template <int W, int CIN, int KIND, bool ZS, int CPI>
 __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col a) {
     using C = ColCfg<W, CIN, KIND>;
     constexpr int MT = C::MT, NR = C::NR, KS = C::KS, WP = C::WP, AP = C::AP, M16 = C::M16;
+    constexpr bool DFT = KIND == 0 || KIND == 1 || KIND == 3, BWD = KIND >= 3;
     const int T = a.nt, n2 = a.n2, npos = a.npos;
     const int ntile = (T + 31) / 32, tpad = 32 * ntile;
     const int tp = tpad + 8;                                   /* pitch of the v' and Ft rows (bf16) */
@@ -94,7 +101,8 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
     const int csub = unit / ntile, tile = unit % ntile;
     const int t = 32 * tile + col;
 
-    for (int i = tid; i < MT * 32; i += 64 * CW) Bl[i] = i < W ? a.bias[i] : 0.f;
+    if constexpr (!BWD)
+        for (int i = tid; i < MT * 32; i += 64 * CW) Bl[i] = i < W ? a.bias[i] : 0.f;
     for (int i = tid; i < MT * 32 * CIN; i += 64 * CW) {
         const int o = i / CIN, k = i % CIN;
         Wl[o * WP + k] = o < W ? a.w[o * CIN + k] : 0.f;
@@ -113,7 +121,7 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
     }
     if constexpr (KIND != 0)
         for (int i = tid; i < CPI * MT * 32 * AP; i += 64 * CW) A6[i] = 0;
-    if constexpr (KIND != 2) {
+    if constexpr (DFT) {
         const int rq = tpad / 8;                               /* 16-byte pieces per row */
         for (int i = tid; i < n16 * 16 * rq; i += 64 * CW)
             *reinterpret_cast<bf16x8 *>(Fl + i / rq * tp + i % rq * 8) = reinterpret_cast<const bf16x8 *>(a.Ft)[i];
@@ -196,14 +204,22 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
             }
         }
         __syncthreads();
-        int bn = b0, pn = pos0;
-        advance(bn, pn, stride);
-        load_v6(bn, pn);
-        load_x(bn, pn);
         int b, pos;
         point(b0, pos0, csub, b, pos);
         const long ob = (long)b * W * cs;
         const unsigned po = 4u * pos * T;
+        float zq[KIND == 3 ? MT : 1][16];                      /* before the next group's loads, which it need not wait for */
+        if constexpr (KIND == 3) {
+            const rsrc_t zb = buf_of(a.zin + ob);
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int r = 0; r < NR; ++r) zq[m][r] = buf_ld(zb, lo, po + (32u * m + 8 * (r / 4) + r % 4) * c4);
+        }
+        int bn = b0, pn = pos0;
+        advance(bn, pn, stride);
+        load_v6(bn, pn);
+        load_x(bn, pn);
         float zr[KIND == 2 ? MT : 1][16];
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
@@ -220,7 +236,11 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
                 if constexpr (KIND != 0) acc[r] += sp[r];
-                acc[r] += Bl[32 * m + 4 * half + 8 * (r / 4) + r % 4];
+                if constexpr (!BWD) acc[r] += Bl[32 * m + 4 * half + 8 * (r / 4) + r % 4];
+                if constexpr (KIND == 3) {
+                    acc[r] *= gelu_d(zq[m][r]);
+                    if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);   /* four GELU' in flight: more spill */
+                }
             }
             /* rows of the lower half-wave: 32 m + 8 (r / 4) + r % 4 */
             auto store = [&](float *base) {
@@ -233,14 +253,16 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
 #pragma unroll
                 for (int r = 0; r < NR; ++r) zr[m][r] = acc[r];
             } else {
-                if (a.act) {
+                if (!BWD && a.act) {
 #pragma unroll
                     for (int r = 0; r < NR; ++r) acc[r] = ZS ? gelu(acc[r]) : gelu_fast(acc[r]);
                 }
                 store(a.out);
-                short *vl = Vl + (csub * M16 * 16 + 32 * m + 4 * half) * tp + t;
+                if constexpr (DFT) {
+                    short *vl = Vl + (csub * M16 * 16 + 32 * m + 4 * half) * tp + t;
 #pragma unroll
-                for (int r = 0; r < NR; ++r) vl[(8 * (r / 4) + r % 4) * tp] = to_bf16(acc[r]);
+                    for (int r = 0; r < NR; ++r) vl[(8 * (r / 4) + r % 4) * tp] = to_bf16(acc[r]);
+                }
             }
         }
         if constexpr (KIND == 2) {
@@ -281,7 +303,7 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
             buf_st(buf_of(a.y + b * 2L * cs), xo, po, ys + x0 + a.q2[half]);
         }
         __syncthreads();
-        if constexpr (KIND != 2) {
+        if constexpr (DFT) {
             constexpr int RND = (CPI * M16 * (CN2_MAX / 16) + CW - 1) / CW;
             const int nt16 = CPI * M16 * n16;
 #pragma unroll
@@ -313,7 +335,7 @@ template <int W, int CIN, int KIND, bool ZS, int CPI> int column_go(const mpc_fn
     const int tp = (a->nt + 31) / 32 * 32 + 8, ht = KIND == 2 ? (a->h + 31) / 32 : 0, n16 = (a->n2 + 15) / 16;
     size_t lds = ((size_t)(C::MT * 32 * (C::WP + 1) + ht * 32 * (W + 4)) * 4 + 15) / 16 * 16;
     if (KIND) lds += (size_t)CPI * C::MT * 32 * C::AP * 2;
-    if (KIND != 2) lds += (size_t)(CPI * C::M16 * 16 + n16 * 16) * tp * 2;
+    if (KIND != 2 && KIND != 4) lds += (size_t)(CPI * C::M16 * 16 + n16 * 16) * tp * 2;
     int dev = 0, ncu = 0, per = 0;
     const void *k = (const void *)k_column<W, CIN, KIND, ZS, CPI>;
     if (hipGetDevice(&dev) != hipSuccess ||
@@ -330,6 +352,7 @@ template <int W, int CIN, int KIND, bool ZS> int column_k(const mpc_fno_col *a, 
     return (a->nt + 31) / 32 <= CW / 2 ? column_go<W, CIN, KIND, ZS, 2>(a, s) : column_go<W, CIN, KIND, ZS, 1>(a, s);
 }
 template <int W> int column_w(const mpc_fno_col *a, hipStream_t s) {
+    if (a->bwd) return a->zin ? column_k<W, W, 3, false>(a, s) : column_k<W, W, 4, false>(a, s);
     if (!a->V6) return column_k<W, 4, 0, false>(a, s);
     if (a->y) return column_k<W, W, 2, false>(a, s);
     return a->zs ? column_k<W, W, 1, true>(a, s) : column_k<W, W, 1, false>(a, s);
@@ -534,14 +557,16 @@ extern "C" int mpc_fno_column_fits(int w, int cin, int nt, int n2, int h) {
 }
 
 extern "C" int mpc_fno_column(const mpc_fno_col *a, void *stream) {
-    if (!a || a->nb <= 0 || a->npos <= 0 || !a->v || !a->w || !a->bias) return MPC_EINVAL;
+    if (!a || a->nb <= 0 || a->npos <= 0 || !a->v || !a->w || (!a->bias && !a->bwd)) return MPC_EINVAL;
     if (!mpc_fno_column_fits(a->width, 4, a->nt, a->n2, a->y ? a->h : 1)) return MPC_EUNSUPP;
     /* byte offsets within a sample's activations and mode rows are 32-bit */
     if ((long)a->width * a->npos * std::max(a->nt, a->n2) > (1L << 29) || (long)a->nb * a->npos > (1L << 30))
         return MPC_EUNSUPP;
     if (a->zs && (!a->V6 || a->y)) return MPC_EINVAL;
     if (a->V6 && !a->Gt) return MPC_EINVAL;
-    if (a->y ? (!a->q1w || !a->q1 || !a->q2w || !a->q2 || !a->x || !a->V6) : (!a->Ft || !a->C1 || !a->out)) return MPC_EINVAL;
+    if (a->bwd) {
+        if (!a->V6 || !a->out || a->zs || a->y || (a->zin && (!a->Ft || !a->C1))) return MPC_EINVAL;
+    } else if (a->y ? (!a->q1w || !a->q1 || !a->q2w || !a->q2 || !a->x || !a->V6) : (!a->Ft || !a->C1 || !a->out)) return MPC_EINVAL;
     hipStream_t s = (hipStream_t)stream;
     switch (a->width) {
     case 8:  return column_w<8>(a, s);

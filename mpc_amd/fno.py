@@ -49,10 +49,11 @@ class MpcPw(C.Structure):
 
 class MpcFnoCol(C.Structure):
     _fields_ = [("nb", C.c_int), ("width", C.c_int), ("npos", C.c_int), ("nt", C.c_int), ("n2", C.c_int),
-                ("act", C.c_int), ("h", C.c_int), ("pad_", C.c_int), ("v", C.c_void_p), ("v_bs", C.c_long),
+                ("act", C.c_int), ("h", C.c_int), ("bwd", C.c_int), ("v", C.c_void_p), ("v_bs", C.c_long),
                 ("V6", C.c_void_p), ("w", C.c_void_p), ("bias", C.c_void_p), ("Gt", C.c_void_p), ("Ft", C.c_void_p),
                 ("zs", C.c_void_p), ("out", C.c_void_p), ("C1", C.c_void_p), ("q1w", C.c_void_p), ("q1", C.c_void_p),
-                ("q2w", C.c_void_p), ("q2", C.c_void_p), ("x", C.c_void_p), ("x_bs", C.c_long), ("y", C.c_void_p)]
+                ("q2w", C.c_void_p), ("q2", C.c_void_p), ("x", C.c_void_p), ("x_bs", C.c_long), ("y", C.c_void_p),
+                ("zin", C.c_void_p)]
 
 
 MIX_BMAX = 8          # samples per mode-mixing launch
@@ -195,13 +196,14 @@ class Ops:
         return d
 
     def column(self, nb, width, npos, nt, n2, v, v_bs, w, bias, V6=None, Gt=None, Ft=None, act=False, zs=None,
-               out=None, C1=None, head=None):
+               out=None, C1=None, head=None, bwd=False, zin=None):
         """the work of every transverse point between two layers' transverse transforms (mpc_fno_column);
-        head: (hidden, Q1, q1, Q2, q2, x, x batch stride, y)"""
+        head: (hidden, Q1, q1, Q2, q2, x, x batch stride, y); bwd, zin: the backward's"""
         a = MpcFnoCol()
         a.nb, a.width, a.npos, a.nt, a.n2, a.act = nb, width, npos, nt, n2, 1 if act else 0
-        a.v, a.v_bs, a.w, a.bias = _ptr(v), v_bs, _ptr(w), _ptr(bias)
-        for name, d in (("V6", V6), ("Gt", Gt), ("Ft", Ft), ("zs", zs), ("out", out), ("C1", C1)):
+        a.v, a.v_bs, a.w, a.bwd = _ptr(v), v_bs, _ptr(w), 1 if bwd else 0
+        for name, d in (("bias", bias), ("V6", V6), ("Gt", Gt), ("Ft", Ft), ("zs", zs), ("out", out), ("C1", C1),
+                        ("zin", zin)):
             setattr(a, name, _ptr(d) if d is not None else None)
         if head is not None:
             a.h, a.x_bs = head[0], head[6]
@@ -335,6 +337,13 @@ class FnoGpu:
             for name, kind, m, k in (("Gyf", 0, cfg.my, cfg.Y), ("Gxf", 0, cfg.mx, cfg.X), ("Gxi", 0, cfg.X, cfg.mx),
                                      ("Gyi", 0, cfg.Y, cfg.my), ("Gt", 2, n2, cfg.T), ("Ft", 3, cfg.T, n2)):
                 self.packed[name, kind] = self.ops.pack(self.mats[name], kind, m, k)
+            # the transposed transforms of the backward
+            for name, m, k in (("Gyf", cfg.my, cfg.Y), ("Gxf", cfg.mx, cfg.X), ("Gxi", cfg.X, cfg.mx), ("Gyi", cfg.Y, cfg.my)):
+                self.packed[name, 1] = self.ops.pack(self.mats[name], 1, m, k)
+            for name, kind, m, k in (("Ft", 2, n2, cfg.T), ("Gt", 3, cfg.T, n2)):
+                t = DArr((m, k))
+                self.ops.transpose(self.mats[name], t, k, m)
+                self.packed[name, kind] = self.ops.pack(t, kind, m, k)
         self.step = 0
         self._buf = {}
 
@@ -563,7 +572,9 @@ class FnoGpu:
         dv = self._b("dv", st["vL"].shape)
         self._pw_bwd_input(self.p["Q1"], dh, dv, H, W, npts, B)
         # Fourier layers, last to first
-        for l in reversed(range(c.layers)):
+        if self.fused:
+            dv = self._layers_bwd_fused(dv, B)
+        for l in reversed(range(0 if self.fused else c.layers)):
             act = l < c.layers - 1
             dz = self._b("dz", dv.shape)
             o.act_bwd(st[f"z{l}"] if act else dv, dv, dz, act)
@@ -575,6 +586,39 @@ class FnoGpu:
         self._pw_bwd_weight(dv, st["x"], self.g["P"], W, c.cin, npts, B)
         o.bias_grad(dv, self.g["bP"], B, W, npts)
         self._st = None
+
+    def _modes_bwd(self, dV6, l, dC1, B):
+        """dC1 = the layer's transposed mode path of dV6; accumulates dRr_l, dRi_l"""
+        c, o, M = self.cfg, self.ops, self.packed
+        W, X, Y, mx, my, mt = c.width, c.X, c.Y, c.mx, c.my, c.mt
+        n2 = 2 * mt
+        dV5, dU = self._b("V5", (B * W, X, my, n2)), self._b("U", (B, W, mx, my, n2))
+        dV3, dV2 = self._b("dV3", (B, W, mx, my, n2)), self._b("V2", (B * W * X, my, n2))
+        o.dft(M["Gyi", 1], dV6, dV5, B * W * X, Y, my, 1, mt, +1, bwd=True)
+        o.dft(M["Gxi", 1], dV5, dU, B * W, X, mx, my, mt, +1, bwd=True)
+        self._mix_bwd(self._st[f"V3{l}"], dU, self.p[f"Rr{l}"], self.p[f"Ri{l}"], dV3, self.g[f"Rr{l}"],
+                      self.g[f"Ri{l}"], B)
+        o.dft(M["Gxf", 1], dV3, dV2, B * W, mx, X, my, mt, -1, bwd=True)
+        o.dft(M["Gyf", 1], dV2, dC1, B * W * X, my, Y, 1, mt, -1, bwd=True)
+
+    def _layers_bwd_fused(self, dz, B):
+        """the Fourier layers' backward from dz of the last one; returns the gradient of the first one's input
+        (in dz's buffer)"""
+        c, o, st, M = self.cfg, self.ops, self._st, self.packed
+        W, npos, n2 = c.width, c.X * c.Y, 2 * c.mt
+        npts = npos * c.T
+        dV6, dC1 = self._b("V6", (B * W * npos, n2)), self._b("C1", (B * W * npos, n2))
+        WT = self._b(f"WT{W}x{W}", (W, W))
+        o.gemm(B * W * npos, n2, c.T, dz, c.T, 1, self.mats["Gt"], 1, c.T, dV6, n2, 1)
+        for l in reversed(range(c.layers)):
+            o.bias_grad(dz, self.g[f"b{l}"], B, W, npts)
+            self._pw_bwd_weight(dz, st[f"v{l}"], self.g[f"W{l}"], W, W, npts, B)
+            self._modes_bwd(dV6, l, dC1, B)
+            o.transpose(self.p[f"W{l}"], WT, W, W)
+            # through the layer, then GELU' and the t-DFT of the one below
+            o.column(B, W, npos, c.T, n2, dz, W * npts, WT, None, V6=dC1, Gt=M["Ft", 2], Ft=M["Gt", 3], out=dz,
+                     C1=dV6, bwd=True, zin=st[f"z{l - 1}"] if l else None)
+        return dz
 
     def loss_and_grad(self, x, tgt):
         """relative L2 loss mean_b |pred-tgt|^2/|tgt|^2; gradients into self.g"""

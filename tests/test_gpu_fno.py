@@ -323,3 +323,41 @@ def test_fused_layers_match_separate_kernels(gpu_lib, W, B, X, Y, T, mx, my, mt,
         assert np.array_equal(a, b)
     a, b = got[True][0].astype(np.float64), got[False][0].astype(np.float64)
     assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b - x[:, :2])
+
+
+@pytest.mark.parametrize("W,B,X,Y,T,mx,my,mt,H", [
+    (32, 2, 16, 16, 256, 8, 8, 32, 64), (8, 1, 11, 9, 37, 5, 4, 3, 8), (16, 3, 12, 10, 100, 6, 5, 24, 32),
+    (64, 1, 9, 8, 64, 4, 8, 16, 64), (32, 1, 7, 5, 132, 7, 5, 9, 16)])
+def test_fused_backward_matches_separate_kernels(gpu_lib, W, B, X, Y, T, mx, my, mt, H):
+    """the backward through the fused kernels against the separate ones on the
+    same network: the gradients of the mode weights, whose operands pass through
+    every fused step below, are the same bits.  The other gradients are FP32 sums
+    over all points whose order may differ: K terms of size s round by about
+    2^-24 sqrt(K) (sqrt(K) s) in all, 2e-5 of a sum of size sqrt(K) s at K = 1e5;
+    1e-4 of the largest one here"""
+    from mpc_amd.fno import FnoConfig, FnoGpu, init_params
+    print(f"case fused backward W={W} B={B} X={X} Y={Y} T={T} modes={mx},{my},{mt} H={H}", flush=True)
+    cfg = FnoConfig(X=X, Y=Y, T=T, width=W, layers=3, mx=mx, my=my, mt=mt, hidden=H)
+    p = init_params(cfg, seed=W + T)
+    rng = np.random.default_rng(T)
+    for k in p:
+        if k[0] == "R":
+            p[k] *= W
+        if k[0] in "bq":
+            p[k] = 0.1 * rng.standard_normal(p[k].shape)
+    x = rng.standard_normal((B, cfg.cin, X, Y, T)).astype(np.float32)
+    tgt = rng.standard_normal((B, 2, X, Y, T)).astype(np.float32)
+    net = FnoGpu(cfg, p)
+    assert net.fused
+    got = {}
+    for fused in (True, False):
+        net.fused = fused
+        loss = net.loss_and_grad(_t(x), _t(tgt))
+        got[fused] = {"loss": np.float64(loss), **{k: g.numpy().astype(np.float64) for k, g in net.g.items()}}
+    assert abs(got[True]["loss"] - got[False]["loss"]) <= 1e-6 * got[False]["loss"]
+    for k, b in got[False].items():
+        a = got[True][k]
+        if k[0] == "R":
+            assert np.array_equal(a, b), k
+        else:
+            assert np.abs(a - b).max() <= 1e-4 * np.abs(b).max(), k
