@@ -155,6 +155,17 @@ int mpc_fno_dft_fits(int m, int kk, int bwd);
 long mpc_fno_pack_bytes(int kind, int m, int kk);
 int  mpc_fno_pack(const float *G, void *out, int kind, int m, int kk, void *stream);
 
+/*
+ * Gradients of a channel map over nb samples of np points: dW[o][i] += sum
+ * d[b][o][p] x[b][i][p] (operands rounded to BF16, FP32 sums) and, unless
+ * NULL, db[o] = sum d[b][o][p].  ws: mpc_fno_wgrad_ws(no, ni, np) bytes of
+ * device memory (MPC_EUNSUPP: not taken; no, ni <= 64, np a multiple of 4; d
+ * and x 16-byte aligned).
+ */
+int  mpc_fno_wgrad(const float *d, const float *x, float *dW, float *db, float *ws, int nb, int no, int ni, long np,
+                   void *stream);
+long mpc_fno_wgrad_ws(int no, int ni, long np);
+
 /* z[b][c][p] += bias[c] (bias may be NULL), then out = GELU(z) if act else z */
 int mpc_fno_bias_act(float *z, const float *bias, float *out, long nb, int nc, long np, int act, void *stream);
 /* dz = dout * GELU'(z) if act else dout */

@@ -84,6 +84,10 @@ __device__ __forceinline__ float2 buf_ld2(rsrc_t r, unsigned lane_off, unsigned 
     const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, lane_off, off, 0);
     return make_float2(__uint_as_float(v[0]), __uint_as_float(v[1]));
 }
+__device__ __forceinline__ float4 buf_ld4(rsrc_t r, unsigned lane_off, unsigned off) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, off, 0);
+    return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
+}
 __device__ __forceinline__ void buf_st(rsrc_t r, unsigned lane_off, unsigned off, float v) {
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, lane_off, off, 0);
 }

@@ -547,6 +547,130 @@ void dft_go(bool tr, const void *G, const float *in, float *out, long nunit, int
     else hipLaunchKernelGGL((k_dft<KS, false>), grid, dim3(256), 0, s, g, in, out, nunit, m, kk, nq, h, sg);
 }
 
+/* ---------------------------------------------------------------------- */
+/* weight and bias gradients of a channel map                              */
+/* ---------------------------------------------------------------------- */
+/*
+ * dW[o][i] = sum over samples and points of d[b][o][p] x[b][i][p] (operands
+ * rounded to BF16, as k_gemm_bf16 does), db[o] = the FP32 sum of d[b][o][p].
+ * Bound by reading d and x once.  Channels lie megabytes apart, so a wave reads
+ * 1 KB of one channel at a time (4 points a lane); read in the operands' order
+ * instead (128 bytes of 32 channels), without the pass through LDS, the same
+ * sums ran at 3.0 TB/s.  At no = ni = 32 and 4.2 M points 206 us (5.2 TB/s); as
+ * a product per sample and a bias kernel 515.
+ * Workgroups walk chunks of 256 points; the next chunk loads under the
+ * products, of which each wave forms 64 points' share.  Each workgroup leaves
+ * its sums in part; k_wgrad_sum adds them.
+ */
+constexpr int WG_WAVES = 4, WG_GRID = 512, WG_MAX = 64, WG_PTS = 256, WG_PITCH = WG_PTS + 8;
+
+template <int OT, int IT>
+__global__ void __launch_bounds__(64 * WG_WAVES, OT + IT == 2 ? 4 : 2)
+k_wgrad(const float *__restrict__ d, const float *__restrict__ x, float *__restrict__ part, int nb, int no, int ni, int np) {
+    constexpr int NE = OT * 32 * (IT * 32 + 1);                /* a workgroup's sums: rows of IT * 32, then db */
+    constexpr int NR = 8 * (OT + IT);                          /* channels a wave loads: wave, wave + 4, ... of d's, then x's */
+    constexpr int BYTES = 32 * (OT + IT) * WG_PITCH * 2, RED = WG_WAVES * OT * IT * 1024 * 4;
+    __shared__ __align__(16) unsigned char smem[BYTES > RED ? BYTES : RED];
+    short *st = reinterpret_cast<short *>(smem);
+    const int lane = threadIdx.x & 63, col = lane & 31, half = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    f32x16 acc[OT][IT] = {};
+    float sum[8 * OT] = {};
+    float4 v[NR];
+    const unsigned np4 = 4u * (unsigned)np;
+    /* channels past no and ni are nobody's: the last one stands in, and its sums are not read */
+    auto load = [&](int b, int p0) {
+        const rsrc_t db = buf_of(d + (long)b * no * np), xb = buf_of(x + (long)b * ni * np);
+        const unsigned p = 4u * min(p0 + 4 * lane, np - 4);
+#pragma unroll
+        for (int i = 0; i < NR; ++i)
+            v[i] = i < 8 * OT ? buf_ld4(db, p, min(wave + 4 * i, no - 1) * np4)
+                              : buf_ld4(xb, p, min(wave + 4 * (i - 8 * OT), ni - 1) * np4);
+    };
+    const int step = WG_PTS * gridDim.x, pend = WG_PTS * ((np + WG_PTS - 1) / WG_PTS);
+    int b = 0, p0 = WG_PTS * blockIdx.x;
+    auto wrap = [&] {
+        while (p0 >= pend) { p0 -= pend; ++b; }
+    };
+    wrap();
+    load(min(b, nb - 1), p0);
+    while (b < nb) {
+        const bool in = p0 + 4 * lane < np;                    /* np is a multiple of 4 */
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            if (!in) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (i < 8 * OT) sum[i < 8 * OT ? i : 0] += (v[i].x + v[i].y) + (v[i].z + v[i].w);
+            *reinterpret_cast<int2 *>(&st[(wave + 4 * i) * WG_PITCH + 4 * lane]) =
+                make_int2(bf16_pair(v[i].x, v[i].y), bf16_pair(v[i].z, v[i].w));
+        }
+        p0 += step;
+        wrap();
+        load(min(b, nb - 1), p0);
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const short *at = st + col * WG_PITCH + 64 * wave + 16 * s + 8 * half;
+            bf16x8 xo[IT];
+#pragma unroll
+            for (int j = 0; j < IT; ++j) xo[j] = *reinterpret_cast<const bf16x8 *>(at + 32 * (OT + j) * WG_PITCH);
+#pragma unroll
+            for (int o = 0; o < OT; ++o) {
+                const bf16x8 dd = *reinterpret_cast<const bf16x8 *>(at + 32 * o * WG_PITCH);
+#pragma unroll
+                for (int j = 0; j < IT; ++j) acc[o][j] = mfma_bf16(dd, xo[j], acc[o][j]);
+            }
+        }
+        __syncthreads();
+    }
+    float *red = reinterpret_cast<float *>(smem), *out = part + (long)blockIdx.x * NE;
+    constexpr int NW = OT * IT * 1024;
+#pragma unroll
+    for (int o = 0; o < OT; ++o)
+#pragma unroll
+        for (int j = 0; j < IT; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                red[wave * NW + (32 * o + drow(r, half)) * IT * 32 + 32 * j + col] = acc[o][j][r];
+#pragma unroll
+    for (int i = 0; i < 8 * OT; ++i) {
+        float t = sum[i];
+#pragma unroll
+        for (int k = 32; k > 0; k >>= 1) t += __shfl_xor(t, k);
+        if (lane == 0) out[NW + wave + 4 * i] = t;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < NW; e += 64 * WG_WAVES)
+        out[e] = (red[e] + red[NW + e]) + (red[2 * NW + e] + red[3 * NW + e]);
+}
+/* dW += and db = the workgroups' sums; 32 entries a block, 32 threads an entry */
+__global__ void __launch_bounds__(1024) k_wgrad_sum(const float *__restrict__ part, int nwg, int oc, int ic,
+                                                    float *__restrict__ dW, float *__restrict__ db, int no, int ni) {
+    __shared__ float red[32][33];
+    const int ne = oc * (ic + 1), e = blockIdx.x * 32 + (threadIdx.x & 31), q = threadIdx.x >> 5;
+    float s = 0.f;
+    if (e < ne)
+        for (int w = q; w < nwg; w += 32) s += part[(long)w * ne + e];
+    red[q][threadIdx.x & 31] = s;
+    __syncthreads();
+    if (q != 0 || e >= ne) return;
+    float t = 0.f;
+#pragma unroll
+    for (int k = 0; k < 32; ++k) t += red[k][threadIdx.x];
+    if (e < oc * ic) {
+        const int o = e / ic, i = e % ic;
+        if (o < no && i < ni) dW[(long)o * ni + i] += t;
+    } else if (db && e - oc * ic < no) {
+        db[e - oc * ic] = t;
+    }
+}
+template <int OT, int IT>
+void wgrad_go(const float *d, const float *x, float *dW, float *db, float *ws, int nb, int no, int ni, long np,
+              hipStream_t s) {
+    const int nwg = (int)std::min((long)WG_GRID, nb * ((np + WG_PTS - 1) / WG_PTS));
+    hipLaunchKernelGGL((k_wgrad<OT, IT>), dim3(nwg), dim3(64 * WG_WAVES), 0, s, d, x, ws, nb, no, ni, (int)np);
+    hipLaunchKernelGGL(k_wgrad_sum, dim3(OT * (IT * 32 + 1)), dim3(1024), 0, s, ws, nwg, OT * 32, IT * 32, dW, db, no, ni);
+}
+
 } // namespace
 
 extern "C" int mpc_sizeof_fno_col(void) { return (int)sizeof(mpc_fno_col); }
@@ -611,5 +735,25 @@ extern "C" int mpc_fno_dft(const void *G, const float *in, float *out, long nsli
     case 4:  dft_go<4>(bwd != 0, G, in, out, nunit, m, kk, nq, h, sg, s); break;
     default: dft_go<8>(bwd != 0, G, in, out, nunit, m, kk, nq, h, sg, s); break;
     }
+    return hipGetLastError() == hipSuccess ? 0 : MPC_EHIP;
+}
+
+extern "C" long mpc_fno_wgrad_ws(int no, int ni, long np) {
+    /* a sample's byte offsets are 32-bit */
+    if (no < 1 || ni < 1 || no > WG_MAX || ni > WG_MAX || np < 4 || np % 4 || np * std::max(no, ni) > (1L << 29))
+        return MPC_EUNSUPP;
+    const long oc = (no + 31) / 32 * 32, ic = (ni + 31) / 32 * 32;
+    return 4 * WG_GRID * oc * (ic + 1);
+}
+
+extern "C" int mpc_fno_wgrad(const float *d, const float *x, float *dW, float *db, float *ws, int nb, int no, int ni,
+                             long np, void *stream) {
+    if (!d || !x || !dW || !ws || nb <= 0 || np <= 0) return MPC_EINVAL;
+    if (mpc_fno_wgrad_ws(no, ni, np) < 0 || (((uintptr_t)d | (uintptr_t)x) & 15)) return MPC_EUNSUPP;
+    hipStream_t s = (hipStream_t)stream;
+    if (no <= 32 && ni <= 32) wgrad_go<1, 1>(d, x, dW, db, ws, nb, no, ni, np, s);
+    else if (no <= 32) wgrad_go<1, 2>(d, x, dW, db, ws, nb, no, ni, np, s);
+    else if (ni <= 32) wgrad_go<2, 1>(d, x, dW, db, ws, nb, no, ni, np, s);
+    else wgrad_go<2, 2>(d, x, dW, db, ws, nb, no, ni, np, s);
     return hipGetLastError() == hipSuccess ? 0 : MPC_EHIP;
 }

@@ -211,6 +211,19 @@ class Ops:
         self.gemm_flops += 2 * nb * width * npos * nt * n2 * ((V6 is not None) + (C1 is not None))
         check(lib().mpc_fno_column(C.cast(C.pointer(a), C.c_void_p), _stream()), "mpc_fno_column")
 
+    def wgrad(self, d, x, dW, db, nout, nin, npts, B):
+        """dW += sum_b d[b] . x[b]^T, db = the sum of d over samples and points"""
+        n = lib().mpc_fno_wgrad_ws(nout, nin, npts)
+        if 0 < n <= 4 * self.ws.numel() and not (d.ptr | x.ptr) % 16:
+            self.gemm_flops += 2 * nout * nin * npts * B
+            check(lib().mpc_fno_wgrad(_ptr(d), _ptr(x), _ptr(dW), _ptr(db), _ptr(self.ws), B, nout, nin, npts,
+                                      _stream()), "mpc_fno_wgrad")
+            return
+        for b in range(B):                        # sizes the kernel does not take
+            self.gemm(nout, nin, npts, d, npts, 1, x, 1, npts, dW, nin, 1, beta=1.0, offA=b * nout * npts,
+                      offB=b * nin * npts)
+        self.bias_grad(d, db, B, nout, npts)
+
     def transpose(self, src, dst, rows, cols):
         check(lib().mpc_fno_transpose(_ptr(src), _ptr(dst), rows, cols, _stream()), "mpc_fno_transpose")
 
@@ -451,12 +464,6 @@ class FnoGpu:
         self.ops.transpose(Wm, WT, nout, nin)
         self.ops.pointwise(dout, nout, WT, nout, 1, dx, nin, B, npts)
 
-    def _pw_bwd_weight(self, dout, x, dW, nout, nin, npts, B):
-        """dW += sum_b dout[b] . x[b]^T"""
-        for b in range(B):
-            self.ops.gemm(nout, nin, npts, dout, npts, 1, x, 1, npts, dW, nin, 1, beta=1.0,
-                          offA=b * nout * npts, offB=b * nin * npts)
-
     # ---- network ---------------------------------------------------------------
     def _fits(self):
         """whether the fused kernels take this network's sizes (they hold a whole t-line of every channel in a
@@ -562,13 +569,11 @@ class FnoGpu:
         for g in self.g.values():
             g.fill(0.0)
         # head
-        self._pw_bwd_weight(dpred, st["h"], self.g["Q2"], c.cout, H, npts, B)
-        o.bias_grad(dpred, self.g["q2"], B, c.cout, npts)
+        o.wgrad(dpred, st["h"], self.g["Q2"], self.g["q2"], c.cout, H, npts, B)
         dh = self._b("dh", st["h"].shape)
         self._pw_bwd_input(self.p["Q2"], dpred, dh, c.cout, H, npts, B)
         o.act_bwd(st["hz"], dh, dh, True)
-        self._pw_bwd_weight(dh, st["vL"], self.g["Q1"], H, W, npts, B)
-        o.bias_grad(dh, self.g["q1"], B, H, npts)
+        o.wgrad(dh, st["vL"], self.g["Q1"], self.g["q1"], H, W, npts, B)
         dv = self._b("dv", st["vL"].shape)
         self._pw_bwd_input(self.p["Q1"], dh, dv, H, W, npts, B)
         # Fourier layers, last to first
@@ -578,13 +583,11 @@ class FnoGpu:
             act = l < c.layers - 1
             dz = self._b("dz", dv.shape)
             o.act_bwd(st[f"z{l}"] if act else dv, dv, dz, act)
-            o.bias_grad(dz, self.g[f"b{l}"], B, W, npts)
-            self._pw_bwd_weight(dz, st[f"v{l}"], self.g[f"W{l}"], W, W, npts, B)
+            o.wgrad(dz, st[f"v{l}"], self.g[f"W{l}"], self.g[f"b{l}"], W, W, npts, B)
             self._pw_bwd_input(self.p[f"W{l}"], dz, dv, W, W, npts, B)
             self._spectral_bwd(dz, l, st[f"V3{l}"], dv)
         # lift (dz0 = dv, no activation)
-        self._pw_bwd_weight(dv, st["x"], self.g["P"], W, c.cin, npts, B)
-        o.bias_grad(dv, self.g["bP"], B, W, npts)
+        o.wgrad(dv, st["x"], self.g["P"], self.g["bP"], W, c.cin, npts, B)
         self._st = None
 
     def _modes_bwd(self, dV6, l, dC1, B):
@@ -611,8 +614,7 @@ class FnoGpu:
         WT = self._b(f"WT{W}x{W}", (W, W))
         o.gemm(B * W * npos, n2, c.T, dz, c.T, 1, self.mats["Gt"], 1, c.T, dV6, n2, 1)
         for l in reversed(range(c.layers)):
-            o.bias_grad(dz, self.g[f"b{l}"], B, W, npts)
-            self._pw_bwd_weight(dz, st[f"v{l}"], self.g[f"W{l}"], W, W, npts, B)
+            o.wgrad(dz, st[f"v{l}"], self.g[f"W{l}"], self.g[f"b{l}"], W, W, npts, B)
             self._modes_bwd(dV6, l, dC1, B)
             o.transpose(self.p[f"W{l}"], WT, W, W)
             # through the layer, then GELU' and the t-DFT of the one below

@@ -361,3 +361,25 @@ def test_fused_backward_matches_separate_kernels(gpu_lib, W, B, X, Y, T, mx, my,
             assert np.array_equal(a, b), k
         else:
             assert np.abs(a - b).max() <= 1e-4 * np.abs(b).max(), k
+
+
+@pytest.mark.parametrize("B,no,ni,npts", [(1, 32, 32, 4096), (3, 32, 4, 1000), (2, 2, 64, 36), (1, 64, 32, 4),
+                                          (2, 64, 64, 132), (2, 8, 8, 2500), (1, 33, 17, 68)])
+def test_weight_gradient_kernel(gpu_lib, B, no, ni, npts):
+    """dW += sum d x^T and db = sum d against float64 on operands rounded to
+    BF16 (d in full for db).  At these sizes a wave sums one piece of at most
+    64 points, and at most 20 additions follow: within 84 * 2^-24 of the sum of
+    the terms' magnitudes"""
+    import torch
+    from mpc_amd.fno import DArr, Ops
+    print(f"case wgrad B={B} no={no} ni={ni} np={npts}", flush=True)
+    rng = np.random.default_rng(npts)
+    d, x = (rng.standard_normal((B, n, npts)).astype(np.float32) for n in (no, ni))
+    w0 = rng.standard_normal((no, ni)).astype(np.float32)
+    o, dW, db = Ops(), DArr.of(w0), DArr((no,)).fill(9.0)
+    o.wgrad(DArr.of(d), DArr.of(x), dW, db, no, ni, npts, B)
+    r = [torch.from_numpy(a).to(torch.bfloat16).double().numpy() for a in (d, x)]
+    tol = 84 * 2.0 ** -24
+    ref, mag = np.einsum("bop,bip->oi", *r), np.einsum("bop,bip->oi", *(np.abs(a) for a in r))
+    assert (np.abs(dW.numpy() - (w0 + ref)) <= tol * (mag + np.abs(w0))).all()
+    assert (np.abs(db.numpy() - d.astype(np.float64).sum((0, 2))) <= tol * np.abs(d).astype(np.float64).sum((0, 2))).all()
