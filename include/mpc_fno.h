@@ -101,7 +101,7 @@ int mpc_fno_mix_bwd(const float *V, const float *dU, const float *Rr, const floa
  * [b][channel][pos][nt]; mode rows V6 and C1 are [b][channel][pos][n2].
  *   V6 == NULL:  the lift, z = w v + bias from the 4 input channels v;
  *   otherwise    z = V6 Gt + w v + bias  (w: width x width, row-major).
- * out receives v' = GELU(z) if act else z, zs (layers only, may be NULL) z.
+ * out receives v' = GELU(z) if act else z, zs (not the lift's; may be NULL) z.
  *   y == NULL:   C1 = v' Ft, the next layer's t-DFT;
  *   otherwise    (no act) the head: y[b][0..2] = q2w GELU(q1w v' + q1) + q2 +
  *                x[b][0..2], h hidden channels, x with batch stride x_bs.
@@ -110,6 +110,13 @@ int mpc_fno_mix_bwd(const float *V, const float *dU, const float *Rr, const floa
  *                result, Gt = Ft^T and Ft = Gt^T; no bias.  With zin, the
  *                pre-activations of the layer below: out = (V6 Gt + w v)
  *                GELU'(zin) and C1 = out Ft; without, out = V6 Gt + w v.
+ *   bwd = 1 with dh (V6 == NULL): through the head.  v is its input v', x is
+ *                dpred[b][0..2], w is q1w transposed: with hz = q1w v' + q1, dh
+ *                = (q2w^T dpred) GELU'(hz) (all h channels), out = w dh, C1 =
+ *                out Ft, dq2w[o][c] += sum dpred[o] GELU(hz)[c] (rounded to
+ *                BF16), dq2[o] = sum dpred[o].  ws: mpc_fno_head_ws(width, h)
+ *                bytes (MPC_EUNSUPP: not taken; width <= 32, h 32 or 64).
+ * zs with y (the same sizes): the same y as z through mpc_fno_pointwise twice.
  * out may be v.  Gt (n2 x nt) and Ft (nt x n2) are given packed (mpc_fno_pack,
  * which rounds them to BF16); V6 and v' are rounded to BF16 as operands of the
  * t-DFTs, as mpc_gemm_bf16 does; the channel maps are FP32.  Supported where
@@ -128,11 +135,13 @@ typedef struct {
     long x_bs;
     float *y;
     const float *zin;
+    float *dh, *ws, *dq2w, *dq2;
 } mpc_fno_col;
 
 int mpc_fno_column(const mpc_fno_col *a, void *stream);
 int mpc_fno_column_fits(int w, int cin, int nt, int n2, int h);
 int mpc_sizeof_fno_col(void);
+long mpc_fno_head_ws(int w, int h);
 
 /*
  * Truncated complex DFT along one axis: the real-block product of G = [cos;

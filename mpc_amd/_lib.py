@@ -117,6 +117,7 @@ def lib() -> C.CDLL:
         "mpc_fno_column": (C.c_int, [vp, vp]),
         "mpc_fno_column_fits": (C.c_int, [C.c_int] * 5),
         "mpc_fno_dft": (C.c_int, [vp, vp, vp, C.c_long, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, vp]),
+        "mpc_fno_head_ws": (C.c_long, [C.c_int] * 2),
         "mpc_fno_wgrad": (C.c_int, [vp, vp, vp, vp, vp, C.c_int, C.c_int, C.c_int, C.c_long, vp]),
         "mpc_fno_wgrad_ws": (C.c_long, [C.c_int, C.c_int, C.c_long]),
         "mpc_fno_pack_bytes": (C.c_long, [C.c_int] * 3),

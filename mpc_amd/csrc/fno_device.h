@@ -25,6 +25,7 @@ __device__ __forceinline__ int bf16_pair(float lo, float hi) {
     p.y = (__bf16)hi;
     return __builtin_bit_cast(int, p);
 }
+__device__ __forceinline__ float bf16_round(float x) { return (float)(__bf16)x; }
 __device__ __forceinline__ bf16x8 bf16_octet(const float (&v)[8]) {
     bf16x8 o;
 #pragma unroll

@@ -30,6 +30,8 @@ namespace {
 constexpr int CW = 8;                  /* waves per workgroup of k_column */
 constexpr int CT_MAX = 256;            /* t points a workgroup covers: CW tiles of 32 */
 constexpr int CN2_MAX = 64;            /* columns of the t-DFT (2 mt) */
+constexpr int CG_MAX = 4096;           /* workgroups of k_column */
+constexpr int CH_MAX = 64;             /* hidden channels of the head */
 
 __device__ __forceinline__ f32x16 mfma_bf16(bf16x8 a, bf16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
@@ -37,9 +39,45 @@ __device__ __forceinline__ f32x16 mfma_bf16(bf16x8 a, bf16x8 b, f32x16 c) {
 __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
+/*
+ * The rows of a 32 x 32 product as the operand of an FP32 product that
+ * contracts over them: step s takes rows 2 s (lower half-wave) and 2 s + 1
+ * (upper), which lie in the registers of two lanes: pairs of registers swap
+ * halves.
+ */
+__device__ __forceinline__ void operand_of(const f32x16 &d, float (&x)[16]) {
+#pragma unroll
+    for (int r = 0; r < 16; r += 2) {
+        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(d[r]), __float_as_uint(d[r + 1]), false, false);
+        const int s = 4 * (r / 4) + (r % 4) / 2;
+        x[s] = __uint_as_float(p[0]);
+        x[s + 2] = __uint_as_float(p[1]);
+    }
+}
 /* row of a 32 x 32 product that register r of a lane in half-wave h holds */
 __device__ __forceinline__ int drow(int r, int h) { return 8 * (r / 4) + 4 * h + r % 4; }
 
+/* dW (oc x ic, of which no x ni are stored) += and db = the sums that nwg workgroups left in part; 32 entries a block, 32 threads an entry */
+__global__ void __launch_bounds__(1024) k_wgrad_sum(const float *__restrict__ part, int nwg, int oc, int ic,
+                                                    float *__restrict__ dW, float *__restrict__ db, int no, int ni) {
+    __shared__ float red[32][33];
+    const int ne = oc * (ic + 1), e = blockIdx.x * 32 + (threadIdx.x & 31), q = threadIdx.x >> 5;
+    float s = 0.f;
+    if (e < ne)
+        for (int w = q; w < nwg; w += 32) s += part[(long)w * ne + e];
+    red[q][threadIdx.x & 31] = s;
+    __syncthreads();
+    if (q != 0 || e >= ne) return;
+    float t = 0.f;
+#pragma unroll
+    for (int k = 0; k < 32; ++k) t += red[k][threadIdx.x];
+    if (e < oc * ic) {
+        const int o = e / ic, i = e % ic;
+        if (o < no && i < ni) dW[(long)o * ni + i] += t;
+    } else if (db && e - oc * ic < no) {
+        db[e - oc * ic] = t;
+    }
+}
 /*
  * k_column<W, CIN, KIND, ZS, CPI>: workgroups walk groups of CPI transverse
  * points (b, pos), grid-stride.  Wave u of a workgroup holds t tile u % ntile
@@ -53,8 +91,17 @@ __device__ __forceinline__ int drow(int r, int h) { return 8 * (r / 4) + 4 * h +
  *           mode path's result, Gt = Ft^T and Wm the transposed channel map of
  *           the layer above, zin this layer's pre-activation
  *   KIND 4, backward through the first layer: V6 Gt + Wm dz only
- * Kinds 0, 1 and 3 then form C1 = v' Ft (3: Ft = Gt^T), from v' rounded to BF16
- * in LDS.  Kind 3 at batch 4 of 64 x 64 x 256 points, width 32, moves 3 streams
+ *   KIND 5, backward through the head: its hidden layer formed again from v as
+ *           KIND 2 does, dh = (Q2^T dpred) GELU'(hz) (stored for Q1's gradient),
+ *           dz = Wm dh with Wm = Q1^T, and the sums of Q2's and q2's gradients
+ * Training's KIND 2 (ZS) also stores v', and its GELU and order of summation
+ * over the hidden channels are the separate kernels' (the products with Q2 go
+ * through the matrix cores), so y keeps its bits.  The last layer, the head and
+ * the way back to dz at batch 4 of 64 x 64 x 256 points, 32 and 64 channels:
+ * 525 + 803 us, bound by the GELUs and the FP32 products; as separate kernels,
+ * which store and read hz, h and dh between them, 2670.
+ * Kinds 0, 1, 3 and 5 then form C1 = v' Ft (3: Ft = Gt^T), from v' rounded to BF16
+ * in LDS (5: as 3).  Kind 3 at batch 4 of 64 x 64 x 256 points, width 32, moves 3 streams
  * of 0.54 GB in 395 us; the four kernels it stands for took 1100.
  * LDS at W = 32, T = 256: Ft 33 KB, v' 17 KB, V6 5 KB, Wm 4 KB: two workgroups
  * (four waves per SIMD) fit on a CU, so one's loads and stores run under the
@@ -71,16 +118,17 @@ template <int W, int CIN, int KIND> struct ColCfg {
     static constexpr int MT = W <= 32 ? 1 : W / 32;            /* 32-row channel tiles */
     static constexpr int NR = W >= 32 ? 16 : W / 2;            /* product registers in use per tile */
     static constexpr int KS = (CIN + 1) / 2;                   /* FP32 product steps of the channel map */
-    static constexpr int WP = CIN + 1;                         /* LDS pitch of the weight rows */
+    static constexpr int WP = (KIND == 5 ? CH_MAX : CIN) + 1;  /* LDS pitch of the weight rows */
     static constexpr int AP = CN2_MAX + 8;                     /* pitch of the staged V6 rows */
     static constexpr int M16 = (W + 15) / 16;                  /* 16-row tiles of the forward t-DFT */
 };
 
 template <int W, int CIN, int KIND, bool ZS, int CPI>
-__global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col a) {
+__global__ void __launch_bounds__(64 * CW, (W <= 32 && KIND != 5 ? 4 : 2)) k_column(mpc_fno_col a) {
     using C = ColCfg<W, CIN, KIND>;
     constexpr int MT = C::MT, NR = C::NR, KS = C::KS, WP = C::WP, AP = C::AP, M16 = C::M16;
-    constexpr bool DFT = KIND == 0 || KIND == 1 || KIND == 3, BWD = KIND >= 3;
+    constexpr bool MODES = KIND != 0 && KIND != 5;             /* takes mode rows V6 */
+    constexpr bool DFT = KIND != 2 && KIND != 4, BWD = KIND >= 3, HEAD = KIND == 2 || KIND == 5;
     const int T = a.nt, n2 = a.n2, npos = a.npos;
     const int ntile = (T + 31) / 32, tpad = 32 * ntile;
     const int tp = tpad + 8;                                   /* pitch of the v' and Ft rows (bf16) */
@@ -90,9 +138,9 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
     float *Bl = reinterpret_cast<float *>(smem);
     float *Wl = Bl + MT * 32;
     float *Ql = Wl + MT * 32 * WP;
-    const int ht = KIND == 2 ? (a.h + 31) / 32 : 0;
+    const int ht = HEAD ? (a.h + 31) / 32 : 0;
     short *A6 = reinterpret_cast<short *>(smem + ((MT * 32 * (WP + 1) + ht * 32 * (W + 4)) * 4 + 15) / 16 * 16);
-    short *Vl = A6 + (KIND ? CPI * MT * 32 * AP : 0);
+    short *Vl = A6 + (MODES ? CPI * MT * 32 * AP : 0);
     short *Fl = Vl + CPI * M16 * 16 * tp;
 
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, half = lane >> 5;
@@ -103,12 +151,19 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
 
     if constexpr (!BWD)
         for (int i = tid; i < MT * 32; i += 64 * CW) Bl[i] = i < W ? a.bias[i] : 0.f;
-    for (int i = tid; i < MT * 32 * CIN; i += 64 * CW) {
-        const int o = i / CIN, k = i % CIN;
-        Wl[o * WP + k] = o < W ? a.w[o * CIN + k] : 0.f;
+    if constexpr (KIND == 5) {                                 /* Q1^T: W x h */
+        for (int i = tid; i < MT * 32 * a.h; i += 64 * CW) {
+            const int o = i / a.h, k = i % a.h;
+            Wl[o * WP + k] = o < W ? a.w[o * a.h + k] : 0.f;
+        }
+    } else {
+        for (int i = tid; i < MT * 32 * CIN; i += 64 * CW) {
+            const int o = i / CIN, k = i % CIN;
+            Wl[o * WP + k] = o < W ? a.w[o * CIN + k] : 0.f;
+        }
     }
     /* q1 | the two rows of Q2 | Q1 */
-    if constexpr (KIND == 2) {
+    if constexpr (HEAD) {
         for (int i = tid; i < ht * 32 * W; i += 64 * CW) {
             const int o = i / W, k = i % W;
             Ql[ht * 96 + o * (W + 1) + k] = o < a.h ? a.q1w[o * W + k] : 0.f;
@@ -119,7 +174,7 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
             Ql[ht * 64 + o] = o < a.h ? a.q2w[a.h + o] : 0.f;
         }
     }
-    if constexpr (KIND != 0)
+    if constexpr (MODES)
         for (int i = tid; i < CPI * MT * 32 * AP; i += 64 * CW) A6[i] = 0;
     if constexpr (DFT) {
         const int rq = tpad / 8;                               /* 16-byte pieces per row */
@@ -127,8 +182,8 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
             *reinterpret_cast<bf16x8 *>(Fl + i / rq * tp + i % rq * 8) = reinterpret_cast<const bf16x8 *>(a.Ft)[i];
     }
     /* the wave's columns of Gt */
-    bf16x8 gB[KIND ? 4 : 1];
-    if constexpr (KIND != 0) {
+    bf16x8 gB[MODES ? 4 : 1];
+    if constexpr (MODES) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) gB[s] = reinterpret_cast<const bf16x8 *>(a.Gt)[(tile * 4 + s) * 64 + lane];
     }
@@ -152,11 +207,11 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
     };
     /* V6 of a group: CPI x W rows of n2 floats (n2 even); 32 threads a row, two floats each */
     constexpr int RPP = 64 * CW / 32, NV = (CPI * W + RPP - 1) / RPP;
-    float2 pre[KIND ? NV : 1];
+    float2 pre[MODES ? NV : 1];
     const int kp = min(tid & 31, n2 / 2 - 1), row0 = tid >> 5;
     const unsigned row4 = 4u * (unsigned)npos * (unsigned)n2;  /* bytes of a channel's mode rows */
     auto load_v6 = [&](int b0, int pos0) {
-        if constexpr (KIND != 0) {
+        if constexpr (MODES) {
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
                 const int r = min(row0 + RPP * i, CPI * W - 1);
@@ -189,14 +244,15 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
             asm volatile("" : "+v"(xn[s]));
             xv[s] = xn[s];
         }
-        if constexpr (KIND != 0) {
+        if constexpr (MODES) {
 #pragma unroll
             for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(pre[i].x), "+v"(pre[i].y));
         }
     };
     arrive();
+    float s2[KIND == 5 ? 2 : 1][2][16] = {}, sb[2] = {};       /* KIND 5: sums of dpred h and dpred */
     while (b0 < a.nb) {
-        if constexpr (KIND != 0) {
+        if constexpr (MODES) {
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
                 const int r = min(row0 + RPP * i, CPI * W - 1);
@@ -216,26 +272,67 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
 #pragma unroll
                 for (int r = 0; r < NR; ++r) zq[m][r] = buf_ld(zb, lo, po + (32u * m + 8 * (r / 4) + r % 4) * c4);
         }
+        float dp[2] = {};
+        if constexpr (KIND == 5) {
+            const rsrc_t db = buf_of(a.x + b * a.x_bs);
+#pragma unroll
+            for (int o = 0; o < 2; ++o) dp[o] = buf_ld(db, to, po + o * c4);
+        }
         int bn = b0, pn = pos0;
         advance(bn, pn, stride);
         load_v6(bn, pn);
         load_x(bn, pn);
         float zr[KIND == 2 ? MT : 1][16];
+        f32x16 dva[KIND == 5 ? MT : 1] = {};
+        if constexpr (KIND == 5) {
+            /* times, waves and points that are only repeated count once */
+            const bool live = wave < CPI * ntile && t < T && (CPI == 1 || (long)b0 * npos + pos0 + csub < (long)a.nb * npos);
+            const float dq0 = live ? bf16_round(dp[0]) : 0.f, dq1 = live ? bf16_round(dp[1]) : 0.f;
+            sb[0] += live ? dp[0] : 0.f;
+            sb[1] += live ? dp[1] : 0.f;
+            const rsrc_t hb = buf_of(a.dh + (long)b * a.h * cs);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                if (q >= ht) break;
+                f32x16 acc = {};
+#pragma unroll
+                for (int s = 0; s < KS; ++s)
+                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(Ql[ht * 96 + (32 * q + col) * (W + 1) + 2 * s + half], xv[s], acc, 0, 0, 0);
+                float xb[16];
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int o = 32 * q + drow(r, half);
+                    const float z = acc[r] + Ql[o], hv = bf16_round(gelu(z));
+                    s2[q][0][r] = fmaf(dq0, hv, s2[q][0][r]);
+                    s2[q][1][r] = fmaf(dq1, hv, s2[q][1][r]);
+                    acc[r] = fmaf(Ql[ht * 64 + o], dp[1], Ql[ht * 32 + o] * dp[0]) * gelu_d(z);
+                    buf_st(hb, lo, po + (32u * q + 8 * (r / 4) + r % 4) * c4, acc[r]);
+                    if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                }
+                operand_of(acc, xb);
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+#pragma unroll
+                    for (int s = 0; s < 16; ++s)
+                        dva[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(Wl[(32 * m + col) * WP + 32 * q + 2 * s + half], xb[s], dva[m], 0, 0, 0);
+            }
+        }
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             f32x16 sp = {}, acc = {};
-            if constexpr (KIND != 0) {
+            if constexpr (KIND == 5) acc = dva[m];
+            if constexpr (MODES) {
 #pragma unroll
                 for (int s = 0; s < 4; ++s)
                     sp = mfma_bf16(*reinterpret_cast<const bf16x8 *>(&A6[((csub * MT + m) * 32 + col) * AP + 16 * s + 8 * half]),
                                    gB[s], sp);
             }
 #pragma unroll
-            for (int s = 0; s < KS; ++s)
+            for (int s = 0; s < (KIND == 5 ? 0 : KS); ++s)
                 acc = __builtin_amdgcn_mfma_f32_32x32x2f32(Wl[(32 * m + col) * WP + 2 * s + half], xv[s], acc, 0, 0, 0);
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
-                if constexpr (KIND != 0) acc[r] += sp[r];
+                if constexpr (MODES) acc[r] += sp[r];
                 if constexpr (!BWD) acc[r] += Bl[32 * m + 4 * half + 8 * (r / 4) + r % 4];
                 if constexpr (KIND == 3) {
                     acc[r] *= gelu_d(zq[m][r]);
@@ -280,6 +377,7 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
                     xb2[s0 + 2] = __uint_as_float(p[1]);
                 }
             float y0 = 0.f, y1 = 0.f;
+            f32x16 ya = {};
             for (int q = 0; q < ht; ++q) {
                 f32x16 acc = {};
 #pragma unroll
@@ -288,17 +386,32 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int o = 32 * q + drow(r, half);
-                    const float hv = gelu_fast(acc[r] + Ql[o]);
-                    y0 = fmaf(Ql[ht * 32 + o], hv, y0);
-                    y1 = fmaf(Ql[ht * 64 + o], hv, y1);
+                    if constexpr (ZS) {
+                        acc[r] = gelu(acc[r] + Ql[o]);
+                    } else {
+                        const float hv = gelu_fast(acc[r] + Ql[o]);
+                        y0 = fmaf(Ql[ht * 32 + o], hv, y0);
+                        y1 = fmaf(Ql[ht * 64 + o], hv, y1);
+                    }
                     /* the rows' LDS operands load where they are used, not all ahead */
                     if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
                 }
+                if constexpr (ZS) {                            /* rows past the second repeat it */
+                    float hb[16];
+                    operand_of(acc, hb);
+#pragma unroll
+                    for (int s = 0; s < 16; ++s)
+                        ya = __builtin_amdgcn_mfma_f32_32x32x2f32(Ql[ht * 32 * (1 + min(col, 1)) + 32 * q + 2 * s + half], hb[s], ya, 0, 0, 0);
+                }
             }
-            /* each half-wave summed its rows of both outputs: the lower one
-             * finishes output 0, the upper one output 1 */
+            /* each half-wave summed its rows of both outputs (ZS: the lower one
+             * all of them): the lower one finishes output 0, the upper output 1 */
+            if constexpr (ZS) {
+                y0 = ya[0];
+                y1 = ya[1];
+            }
             const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(y0), __float_as_uint(y1), false, false);
-            const float ys = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+            const float ys = ZS ? __uint_as_float(p[0]) : __uint_as_float(p[0]) + __uint_as_float(p[1]);
             const float x0 = buf_ld(buf_of(a.x + b * a.x_bs), xo, po);
             buf_st(buf_of(a.y + b * 2L * cs), xo, po, ys + x0 + a.q2[half]);
         }
@@ -328,13 +441,45 @@ __global__ void __launch_bounds__(64 * CW, W <= 32 ? 4 : 2) k_column(mpc_fno_col
         b0 = bn;
         pos0 = pn;
     }
+    if constexpr (KIND == 5) {
+        /* this workgroup's [2][h] sums and the two of dpred: over a half-wave's times, then the waves in order */
+        float *red = reinterpret_cast<float *>(smem);          /* [CW][2 CH_MAX + 2]; the last products' barrier is behind */
+        __syncthreads();
+        constexpr int NE = 2 * CH_MAX + 2;
+        auto lanes = [&](float v) {
+#pragma unroll
+            for (int k = 16; k > 0; k >>= 1) v += __shfl_xor(v, k);
+            return v;
+        };
+#pragma unroll
+        for (int o = 0; o < 2; ++o) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float v = lanes(s2[q][o][r]);
+                    if (col == 0) red[wave * NE + o * CH_MAX + 32 * q + drow(r, half)] = v;
+                }
+            const float v = lanes(sb[o]);
+            if (lane == 0) red[wave * NE + 2 * CH_MAX + o] = v;
+        }
+        __syncthreads();
+        const int ne = 2 * (a.h + 1);
+        for (int e = tid; e < ne; e += 64 * CW) {
+            const int src = e < 2 * a.h ? e / a.h * CH_MAX + e % a.h : 2 * CH_MAX + e - 2 * a.h;
+            float v = 0.f;
+#pragma unroll
+            for (int w = 0; w < CW; ++w) v += red[w * NE + src];
+            a.ws[(long)blockIdx.x * ne + e] = v;
+        }
+    }
 }
 
 template <int W, int CIN, int KIND, bool ZS, int CPI> int column_go(const mpc_fno_col *a, hipStream_t s) {
     using C = ColCfg<W, CIN, KIND>;
-    const int tp = (a->nt + 31) / 32 * 32 + 8, ht = KIND == 2 ? (a->h + 31) / 32 : 0, n16 = (a->n2 + 15) / 16;
+    const int tp = (a->nt + 31) / 32 * 32 + 8, ht = KIND == 2 || KIND == 5 ? (a->h + 31) / 32 : 0, n16 = (a->n2 + 15) / 16;
     size_t lds = ((size_t)(C::MT * 32 * (C::WP + 1) + ht * 32 * (W + 4)) * 4 + 15) / 16 * 16;
-    if (KIND) lds += (size_t)CPI * C::MT * 32 * C::AP * 2;
+    if (KIND != 0 && KIND != 5) lds += (size_t)CPI * C::MT * 32 * C::AP * 2;
     if (KIND != 2 && KIND != 4) lds += (size_t)(CPI * C::M16 * 16 + n16 * 16) * tp * 2;
     int dev = 0, ncu = 0, per = 0;
     const void *k = (const void *)k_column<W, CIN, KIND, ZS, CPI>;
@@ -343,8 +488,11 @@ template <int W, int CIN, int KIND, bool ZS, int CPI> int column_go(const mpc_fn
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, 64 * CW, lds) != hipSuccess || per < 1)
         return MPC_EHIP;
     const long ngrp = ((long)a->nb * a->npos + CPI - 1) / CPI;
-    const unsigned grid = (unsigned)std::min(ngrp, (long)ncu * per);
+    const unsigned grid = (unsigned)std::min(ngrp, std::min((long)ncu * per, (long)CG_MAX));
     hipLaunchKernelGGL((k_column<W, CIN, KIND, ZS, CPI>), dim3(grid), dim3(64 * CW), lds, s, *a);
+    if (KIND == 5)
+        hipLaunchKernelGGL(k_wgrad_sum, dim3((2 * (a->h + 1) + 31) / 32), dim3(1024), 0, s, a->ws, (int)grid, 2, a->h,
+                           a->dq2w, a->dq2, 2, a->h);
     return hipGetLastError() == hipSuccess ? 0 : MPC_EHIP;
 }
 /* short lines (at most CW/2 t tiles): two points at a time, so that no wave idles */
@@ -352,6 +500,10 @@ template <int W, int CIN, int KIND, bool ZS> int column_k(const mpc_fno_col *a, 
     return (a->nt + 31) / 32 <= CW / 2 ? column_go<W, CIN, KIND, ZS, 2>(a, s) : column_go<W, CIN, KIND, ZS, 1>(a, s);
 }
 template <int W> int column_w(const mpc_fno_col *a, hipStream_t s) {
+    if constexpr (W <= 32) {
+        if (a->dh) return column_k<W, W, 5, false>(a, s);
+        if (a->y && a->zs) return column_k<W, W, 2, true>(a, s);
+    }
     if (a->bwd) return a->zin ? column_k<W, W, 3, false>(a, s) : column_k<W, W, 4, false>(a, s);
     if (!a->V6) return column_k<W, 4, 0, false>(a, s);
     if (a->y) return column_k<W, W, 2, false>(a, s);
@@ -642,27 +794,6 @@ k_wgrad(const float *__restrict__ d, const float *__restrict__ x, float *__restr
     for (int e = threadIdx.x; e < NW; e += 64 * WG_WAVES)
         out[e] = (red[e] + red[NW + e]) + (red[2 * NW + e] + red[3 * NW + e]);
 }
-/* dW += and db = the workgroups' sums; 32 entries a block, 32 threads an entry */
-__global__ void __launch_bounds__(1024) k_wgrad_sum(const float *__restrict__ part, int nwg, int oc, int ic,
-                                                    float *__restrict__ dW, float *__restrict__ db, int no, int ni) {
-    __shared__ float red[32][33];
-    const int ne = oc * (ic + 1), e = blockIdx.x * 32 + (threadIdx.x & 31), q = threadIdx.x >> 5;
-    float s = 0.f;
-    if (e < ne)
-        for (int w = q; w < nwg; w += 32) s += part[(long)w * ne + e];
-    red[q][threadIdx.x & 31] = s;
-    __syncthreads();
-    if (q != 0 || e >= ne) return;
-    float t = 0.f;
-#pragma unroll
-    for (int k = 0; k < 32; ++k) t += red[k][threadIdx.x];
-    if (e < oc * ic) {
-        const int o = e / ic, i = e % ic;
-        if (o < no && i < ni) dW[(long)o * ni + i] += t;
-    } else if (db && e - oc * ic < no) {
-        db[e - oc * ic] = t;
-    }
-}
 template <int OT, int IT>
 void wgrad_go(const float *d, const float *x, float *dW, float *db, float *ws, int nb, int no, int ni, long np,
               hipStream_t s) {
@@ -680,17 +811,32 @@ extern "C" int mpc_fno_column_fits(int w, int cin, int nt, int n2, int h) {
            n2 <= CN2_MAX && h >= 1 && h <= 64 && (h & (h - 1)) == 0;
 }
 
+/* dh is stored in whole tiles of 32 hidden channels; at width 64 the sums and
+ * operands of kind 5 exceed the registers (61 spills) */
+extern "C" long mpc_fno_head_ws(int w, int h) {
+    return w > 32 || h < 1 || h > CH_MAX || h % 32 ? MPC_EUNSUPP : 4L * CG_MAX * 2 * (h + 1);
+}
+
 extern "C" int mpc_fno_column(const mpc_fno_col *a, void *stream) {
     if (!a || a->nb <= 0 || a->npos <= 0 || !a->v || !a->w || (!a->bias && !a->bwd)) return MPC_EINVAL;
-    if (!mpc_fno_column_fits(a->width, 4, a->nt, a->n2, a->y ? a->h : 1)) return MPC_EUNSUPP;
+    if (!mpc_fno_column_fits(a->width, 4, a->nt, a->n2, a->y || a->dh ? a->h : 1)) return MPC_EUNSUPP;
     /* byte offsets within a sample's activations and mode rows are 32-bit */
     if ((long)a->width * a->npos * std::max(a->nt, a->n2) > (1L << 29) || (long)a->nb * a->npos > (1L << 30))
         return MPC_EUNSUPP;
-    if (a->zs && (!a->V6 || a->y)) return MPC_EINVAL;
-    if (a->V6 && !a->Gt) return MPC_EINVAL;
-    if (a->bwd) {
+    if (a->zs && !a->V6) return MPC_EINVAL;
+    if ((a->dh || (a->y && a->zs)) && mpc_fno_head_ws(a->width, a->h) < 0) return MPC_EUNSUPP;
+    if (a->dh) {
+        if ((long)a->h * a->npos * a->nt > (1L << 29)) return MPC_EUNSUPP;
+        if (!a->bwd || a->V6 || a->zin || a->y || !a->q1w || !a->q1 || !a->q2w || !a->x || !a->out || !a->Ft || !a->C1 ||
+            !a->ws || !a->dq2w || !a->dq2)
+            return MPC_EINVAL;
+    } else if (a->V6 && !a->Gt) {
+        return MPC_EINVAL;
+    } else if (a->bwd) {
         if (!a->V6 || !a->out || a->zs || a->y || (a->zin && (!a->Ft || !a->C1))) return MPC_EINVAL;
-    } else if (a->y ? (!a->q1w || !a->q1 || !a->q2w || !a->q2 || !a->x || !a->V6) : (!a->Ft || !a->C1 || !a->out)) return MPC_EINVAL;
+    } else if (a->y ? (!a->q1w || !a->q1 || !a->q2w || !a->q2 || !a->x || !a->V6) : (!a->Ft || !a->C1 || !a->out)) {
+        return MPC_EINVAL;
+    }
     hipStream_t s = (hipStream_t)stream;
     switch (a->width) {
     case 8:  return column_w<8>(a, s);

@@ -53,7 +53,7 @@ class MpcFnoCol(C.Structure):
                 ("V6", C.c_void_p), ("w", C.c_void_p), ("bias", C.c_void_p), ("Gt", C.c_void_p), ("Ft", C.c_void_p),
                 ("zs", C.c_void_p), ("out", C.c_void_p), ("C1", C.c_void_p), ("q1w", C.c_void_p), ("q1", C.c_void_p),
                 ("q2w", C.c_void_p), ("q2", C.c_void_p), ("x", C.c_void_p), ("x_bs", C.c_long), ("y", C.c_void_p),
-                ("zin", C.c_void_p)]
+                ("zin", C.c_void_p), ("dh", C.c_void_p), ("ws", C.c_void_p), ("dq2w", C.c_void_p), ("dq2", C.c_void_p)]
 
 
 MIX_BMAX = 8          # samples per mode-mixing launch
@@ -211,6 +211,17 @@ class Ops:
         self.gemm_flops += 2 * nb * width * npos * nt * n2 * ((V6 is not None) + (C1 is not None))
         check(lib().mpc_fno_column(C.cast(C.pointer(a), C.c_void_p), _stream()), "mpc_fno_column")
 
+    def head_bwd(self, nb, width, npos, nt, n2, hidden, v, Q1, q1, Q2, Q1T, dpred, Ft, dh, out, C1, dQ2, dq2):
+        """the backward through the projection head (mpc_fno_column's dh form)"""
+        a = MpcFnoCol()
+        a.nb, a.width, a.npos, a.nt, a.n2, a.h, a.bwd = nb, width, npos, nt, n2, hidden, 1
+        a.v, a.v_bs, a.x_bs = _ptr(v), width * npos * nt, 2 * npos * nt
+        for name, d in (("q1w", Q1), ("q1", q1), ("q2w", Q2), ("w", Q1T), ("x", dpred), ("Ft", Ft), ("dh", dh),
+                        ("out", out), ("C1", C1), ("ws", self.ws), ("dq2w", dQ2), ("dq2", dq2)):
+            setattr(a, name, _ptr(d))
+        self.gemm_flops += 2 * nb * width * npos * nt * n2 + 4 * nb * hidden * npos * nt
+        check(lib().mpc_fno_column(C.cast(C.pointer(a), C.c_void_p), _stream()), "mpc_fno_column")
+
     def wgrad(self, d, x, dW, db, nout, nin, npts, B):
         """dW += sum_b d[b] . x[b]^T, db = the sum of d over samples and points"""
         n = lib().mpc_fno_wgrad_ws(nout, nin, npts)
@@ -344,6 +355,8 @@ class FnoGpu:
         self.v = {k: zeros(v.shape) for k, v in self.p.items()}
         self.mats = {k: DArr.of(v) for k, v in dft_mats(cfg).items()}
         self.fused = self._fits()
+        # whether training's head is fused too
+        self.fused_head = 0 < lib().mpc_fno_head_ws(cfg.width, cfg.hidden) <= 4 * self.ops.ws.numel()
         self.packed = {}
         if self.fused:
             n2 = 2 * cfg.mt
@@ -469,7 +482,8 @@ class FnoGpu:
         """whether the fused kernels take this network's sizes (they hold a whole t-line of every channel in a
         workgroup); larger ones run the separate kernels"""
         c, L = self.cfg, lib()
-        return bool(c.cout == 2 and L.mpc_fno_column_fits(c.width, c.cin, c.T, 2 * c.mt, c.hidden) and
+        # byte offsets within a sample are 32-bit
+        return bool(c.cout == 2 and max(c.width, c.hidden) * c.X * c.Y * max(c.T, 2 * c.mt) <= 1 << 29 and L.mpc_fno_column_fits(c.width, c.cin, c.T, 2 * c.mt, c.hidden) and
                     all(L.mpc_fno_dft_fits(m, k, bwd) for bwd in (0, 1)
                         for m, k in ((c.my, c.Y), (c.mx, c.X), (c.X, c.mx), (c.Y, c.my))))
 
@@ -503,8 +517,13 @@ class FnoGpu:
             V3 = self._b(f"V3{l}", (B, W, c.mx, c.my, n2)) if keep else None
             self._modes_fwd(C1, l, V6, V3, B)
             args = (B, W, npos, c.T, n2, v, W * npts, self.p[f"W{l}"], self.p[f"b{l}"], V6, M["Gt", 2], M["Ft", 3])
-            if last and not keep:
-                o.column(*args, head=(H, self.p["Q1"], self.p["q1"], self.p["Q2"], self.p["q2"], x, c.cin * npts, y))
+            if last and (not keep or self.fused_head):
+                vL = self._b(f"v{l + 1}", shp) if keep else None
+                o.column(*args, zs=vL,
+                         head=(H, self.p["Q1"], self.p["q1"], self.p["Q2"], self.p["q2"], x, c.cin * npts, y))
+                if keep:
+                    st[f"v{l}"], st[f"V3{l}"], st["vL"] = v, V3, vL
+                    self._st = st
                 return y
             z = self._b(f"z{l}", shp) if keep and not last else None
             # in place without keep (a point's channels are read before they are
@@ -569,8 +588,19 @@ class FnoGpu:
         for g in self.g.values():
             g.fill(0.0)
         # head
+        dh = self._b("dh", (B, H, c.X, c.Y, c.T))
+        if self.fused and self.fused_head:
+            Q1T, n2, npos = self._b(f"WT{H}x{W}", (W, H)), 2 * c.mt, c.X * c.Y
+            o.transpose(self.p["Q1"], Q1T, H, W)
+            dz, dV6 = self._b("dv", st["vL"].shape), self._b("V6", (B * W * npos, n2))
+            o.head_bwd(B, W, npos, c.T, n2, H, st["vL"], self.p["Q1"], self.p["q1"], self.p["Q2"], Q1T, dpred,
+                       self.packed["Gt", 3], dh, dz, dV6, self.g["Q2"], self.g["q2"])
+            o.wgrad(dh, st["vL"], self.g["Q1"], self.g["q1"], H, W, npts, B)
+            dv = self._layers_bwd_fused(dz, dV6, B)
+            o.wgrad(dv, st["x"], self.g["P"], self.g["bP"], W, c.cin, npts, B)
+            self._st = None
+            return
         o.wgrad(dpred, st["h"], self.g["Q2"], self.g["q2"], c.cout, H, npts, B)
-        dh = self._b("dh", st["h"].shape)
         self._pw_bwd_input(self.p["Q2"], dpred, dh, c.cout, H, npts, B)
         o.act_bwd(st["hz"], dh, dh, True)
         o.wgrad(dh, st["vL"], self.g["Q1"], self.g["q1"], H, W, npts, B)
@@ -578,7 +608,9 @@ class FnoGpu:
         self._pw_bwd_input(self.p["Q1"], dh, dv, H, W, npts, B)
         # Fourier layers, last to first
         if self.fused:
-            dv = self._layers_bwd_fused(dv, B)
+            dV6 = self._b("V6", (B * W * c.X * c.Y, 2 * c.mt))
+            o.gemm(B * W * c.X * c.Y, 2 * c.mt, c.T, dv, c.T, 1, self.mats["Gt"], 1, c.T, dV6, 2 * c.mt, 1)
+            dv = self._layers_bwd_fused(dv, dV6, B)
         for l in reversed(range(0 if self.fused else c.layers)):
             act = l < c.layers - 1
             dz = self._b("dz", dv.shape)
@@ -604,15 +636,14 @@ class FnoGpu:
         o.dft(M["Gxf", 1], dV3, dV2, B * W, mx, X, my, mt, -1, bwd=True)
         o.dft(M["Gyf", 1], dV2, dC1, B * W * X, my, Y, 1, mt, -1, bwd=True)
 
-    def _layers_bwd_fused(self, dz, B):
-        """the Fourier layers' backward from dz of the last one; returns the gradient of the first one's input
+    def _layers_bwd_fused(self, dz, dV6, B):
+        """the Fourier layers' backward from dz of the last one and its t-DFT dV6; returns the gradient of the first one's input
         (in dz's buffer)"""
         c, o, st, M = self.cfg, self.ops, self._st, self.packed
         W, npos, n2 = c.width, c.X * c.Y, 2 * c.mt
         npts = npos * c.T
-        dV6, dC1 = self._b("V6", (B * W * npos, n2)), self._b("C1", (B * W * npos, n2))
+        dC1 = self._b("C1", (B * W * npos, n2))
         WT = self._b(f"WT{W}x{W}", (W, W))
-        o.gemm(B * W * npos, n2, c.T, dz, c.T, 1, self.mats["Gt"], 1, c.T, dV6, n2, 1)
         for l in reversed(range(c.layers)):
             o.wgrad(dz, st[f"v{l}"], self.g[f"W{l}"], self.g[f"b{l}"], W, W, npts, B)
             self._modes_bwd(dV6, l, dC1, B)

@@ -327,7 +327,8 @@ def test_fused_layers_match_separate_kernels(gpu_lib, W, B, X, Y, T, mx, my, mt,
 
 @pytest.mark.parametrize("W,B,X,Y,T,mx,my,mt,H", [
     (32, 2, 16, 16, 256, 8, 8, 32, 64), (8, 1, 11, 9, 37, 5, 4, 3, 8), (16, 3, 12, 10, 100, 6, 5, 24, 32),
-    (64, 1, 9, 8, 64, 4, 8, 16, 64), (32, 1, 7, 5, 132, 7, 5, 9, 16)])
+    (64, 1, 9, 8, 64, 4, 8, 16, 64), (32, 1, 7, 5, 132, 7, 5, 9, 16), (16, 1, 7, 5, 100, 5, 4, 24, 32),
+    (8, 3, 5, 3, 31, 3, 2, 7, 64)])
 def test_fused_backward_matches_separate_kernels(gpu_lib, W, B, X, Y, T, mx, my, mt, H):
     """the backward through the fused kernels against the separate ones on the
     same network: the gradients of the mode weights, whose operands pass through
