@@ -138,16 +138,18 @@ template <class G> __device__ __forceinline__ void tline_flush_rho(double rmax, 
 
 /*
  * Whether a persistent workgroup loads its next line under the current one's
- * transforms (and keeps the Omega grid in registers).  In FP32 those 24
- * registers are worth more as a third wave per SIMD, whose work covers the
- * loads: 256x256x2048 1.10 -> 1.03 ms, 128x128x512 60 -> 56 us.  A 4096-point
- * line's workgroup of eight waves leaves room for two per SIMD only (160
- * against 175 us at 64x64x4096), and FP64 for one.
+ * transforms (and keeps the Omega grid in registers).  Those registers (24 in
+ * FP32, 48 in FP64) are worth more as another wave per SIMD, whose work covers
+ * the loads: three instead of two in FP32 (256x256x2048 1.10 -> 1.03 ms,
+ * 128x128x512 60 -> 56 us), two instead of one in FP64 (2.55 -> 1.88 ms, 137 ->
+ * 108 us, 64x64x512 39 -> 31 us; now at least level with the per-group form up
+ * to 2048 points).  An FP32 4096-point line's workgroup of eight waves leaves
+ * room for two per SIMD only (160 against 175 us at 64x64x4096).
  */
-template <class T, class G, bool PERSIST> constexpr bool TLinePre = PERSIST && (sizeof(T) == 8 || G::NT == 4096);
+template <class T, class G, bool PERSIST> constexpr bool TLinePre = PERSIST && sizeof(T) == 4 && G::NT == 4096;
 /* waves per SIMD the kernel is held to */
 template <class T, class G, bool PERSIST>
-constexpr int TLineWaves = sizeof(T) == 8 ? 1 : TLinePre<T, G, PERSIST> ? 2 : 3;
+constexpr int TLineWaves = sizeof(T) == 8 ? (PERSIST ? 2 : 1) : TLinePre<T, G, PERSIST> ? 2 : 3;
 
 /* the work of one workgroup: line groups grp, grp + gstride, ... of the
  * field a describes (one group unless PERSIST); its plasma maximum goes to
