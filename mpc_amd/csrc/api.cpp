@@ -212,6 +212,14 @@ extern "C" int mpc_create(const mpc_params *p, int precision, mpc_ctx **out) {
     }
     if (!rc) rc = ctx_set_params(c, p);
     if (rc) { mpc_destroy(c); return rc; }
+    /* until tuned: persistent axis sweeps for lines from 128 points on, whose
+     * tables are worth keeping from tile to tile (x / y sweeps, FP32: 128x128x512
+     * 32 / 31 -> 28 / 27 us, 192x192x1024 156 / 165 -> 120 / 132, 256x256x2048
+     * 435 / 516 -> 374 / 437; FP64 256x256x2048 800 / 904 -> 795 / 857), a
+     * workgroup per tile for shorter ones (FP64 64x64x512 16.1 / 14.4 against
+     * 17.5 / 16.8, 64x64x4096 89 / 83 against 86 / 90) */
+    c->avar = c->nx >= 128 ? 16 : 0;
+    c->avar_y = c->ny >= 128 ? 16 : 0;
     if (const char *e = getenv("MPC_TLINE_VARIANT")) c->tvar = std::max(0, std::min(tline_variants() - 1, atoi(e)));
     if (const char *e = getenv("MPC_AXIS_VARIANT")) c->avar = c->avar_y = std::max(0, std::min(axis_variants() - 1, atoi(e)));
     *out = c;
