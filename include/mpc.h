@@ -198,7 +198,7 @@ int  mpc_variant_counts(int *tline_variants, int *axis_variants);
  * Batched runs (no counterpart in the reference): pulses of uneven grids,
  * energies and media, one context each (same precision, steps_per_pass and
  * npasses), advance together.  Pulses of one size class are split into
- * launch groups of at most 256 MB of fields, and every sweep of a step is one
+ * launch groups of at most 192 MB of fields, and every sweep of a step is one
  * launch per group.  Within a pass each group runs all its sweeps before the
  * next group starts, so a pulse's sweep finds part of what its previous
  * sweep wrote still in the last-level cache (when the sweep kinds group the
