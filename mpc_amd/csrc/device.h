@@ -573,7 +573,7 @@ __device__ __forceinline__ void plasma_line(const cx<T> (&A)[G::E], int tid, dou
     line_sync<G::WAVE>();         /* the LDS may still be read by the caller's last exchange */
 #pragma unroll
     for (int m = 0; m < E; ++m) {
-        const int k = padp_tm<G>(tid, m);                  /* element tid + TPL*m, swizzled */
+        const int k = padp_tm<G>(tid, m);                  /* where element tid + TPL*m lies */
         PlasmaElem<T> pe;
         pe.set(A[m].re, A[m].im, pk);
         T tc;

@@ -16,7 +16,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 /* FP32 -> BF16, round to nearest even (v_cvt_pk_bf16_f32) */
-__device__ __forceinline__ __bf16 bf16_of(float f) { return (__bf16)f; }
 __device__ __forceinline__ short to_bf16(float f) { return __builtin_bit_cast(short, (__bf16)f); }
 __device__ __forceinline__ int bf16_pair(float lo, float hi) {
     typedef __bf16 v2 __attribute__((ext_vector_type(2)));
