@@ -178,6 +178,26 @@ static int ctx_set_params(mpc_ctx *c, const mpc_params *p) {
     return c->prec == MPC_F32 ? setup_tables<float>(c) : setup_tables<double>(c);
 }
 
+/*
+ * The x/y sweeps' variant until tuned: persistent workgroups (16), which keep a
+ * line's tables from tile to tile, where they measured faster than a workgroup
+ * per tile (0).  Sum of an x and a y sweep on n x n x nt points, 0 -> 16, in us:
+ *   FP32  128: nt 256 36 -> 34, 512 63 -> 56, 2048 186 -> 181, 4096 496 -> 397;
+ *         192: 256 93 -> 75, 1024 322 -> 251; 256: 256 117 -> 107, 2048 956 -> 820;
+ *         512: 256 727 -> 1463, 512 1465 -> 2913 (129 registers spilled).
+ *   FP64  128: 256 57 -> 51, 512 96 -> 89, 1024 169 -> 170, 2048 396 -> 408, 4096
+ *         818 -> 865 (from 1024 points on the field exceeds the last-level cache);
+ *         192: 256 149 -> 134, 1024 561 -> 523, 2048 1127 -> 1017;
+ *         256: 256 174 -> 179, 512 408 -> 407, 1024 836 -> 813, 2048 1713 -> 1657;
+ *         512: 256 1084 -> 1219, 512 2187 -> 2432 (44 spilled).
+ * Shorter lines lose in FP64 (64: nt 512 31 -> 34) and gain nothing in FP32.
+ */
+static int default_axis_variant(int precision, int n, int nt) {
+    const bool persist = precision == MPC_F32 ? n >= 128 && n <= 256
+                                              : n == 192 || (n == 128 && nt <= 512) || (n == 256 && nt >= 512);
+    return persist ? 16 : 0;
+}
+
 extern "C" int mpc_create(const mpc_params *p, int precision, mpc_ctx **out) {
     if (!out) return MPC_EINVAL;
     *out = nullptr;
@@ -212,14 +232,8 @@ extern "C" int mpc_create(const mpc_params *p, int precision, mpc_ctx **out) {
     }
     if (!rc) rc = ctx_set_params(c, p);
     if (rc) { mpc_destroy(c); return rc; }
-    /* until tuned: persistent axis sweeps for lines from 128 points on, whose
-     * tables are worth keeping from tile to tile (x / y sweeps, FP32: 128x128x512
-     * 32 / 31 -> 28 / 27 us, 192x192x1024 156 / 165 -> 120 / 132, 256x256x2048
-     * 435 / 516 -> 374 / 437; FP64 256x256x2048 800 / 904 -> 795 / 857), a
-     * workgroup per tile for shorter ones (FP64 64x64x512 16.1 / 14.4 against
-     * 17.5 / 16.8, 64x64x4096 89 / 83 against 86 / 90) */
-    c->avar = c->nx >= 128 ? 16 : 0;
-    c->avar_y = c->ny >= 128 ? 16 : 0;
+    c->avar = default_axis_variant(precision, c->nx, c->nt);
+    c->avar_y = default_axis_variant(precision, c->ny, c->nt);
     if (const char *e = getenv("MPC_TLINE_VARIANT")) c->tvar = std::max(0, std::min(tline_variants() - 1, atoi(e)));
     if (const char *e = getenv("MPC_AXIS_VARIANT")) c->avar = c->avar_y = std::max(0, std::min(axis_variants() - 1, atoi(e)));
     *out = c;
