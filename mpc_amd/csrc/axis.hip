@@ -99,7 +99,7 @@ __device__ __forceinline__ void axis_work(const AArgs<T> &a, long lin, long lstr
     int tid = tid0, gcol = gcol0;
     auto fft = [&](cx<T>(&x)[E], auto dir) {
         constexpr int DIR = decltype(dir)::value;
-        if constexpr (PERSIST) CO::template fft<DIR, 0>(x, tid, lds + gcol, G, twc);
+        if constexpr (PERSIST) CO::template fft<DIR>(x, tid, lds + gcol, G, twc);
         else line_fft<T, N, PL, DIR>(x, tid, lds + gcol, G, a.tw);
     };
 
@@ -211,7 +211,7 @@ k_axis_batch_p(const AArgs<T> *__restrict__ d, const long *__restrict__ tstart, 
     int tid = tid0, gcol = gcol0;
     auto fft = [&](cx<T>(&x)[E], auto dir) {
         constexpr int DIR = decltype(dir)::value;
-        CO::template fft<DIR, 0>(x, tid, lds + gcol, G, twc);
+        CO::template fft<DIR>(x, tid, lds + gcol, G, twc);
     };
 
     cx<T> nxt[E], pn = mk((T)1, (T)0);
@@ -308,7 +308,7 @@ k_axis_richardson(AArgs<T> a, const cx<T> *__restrict__ c1, double *__restrict__
     int tid = tid0, gcol = gcol0;
     auto fft = [&](cx<T>(&x)[E], auto dir) {
         constexpr int DIR = decltype(dir)::value;
-        if constexpr (PERSIST) CO::template fft<DIR, 0>(x, tid, lds + gcol, G, twc);
+        if constexpr (PERSIST) CO::template fft<DIR>(x, tid, lds + gcol, G, twc);
         else line_fft<T, N, PL, DIR>(x, tid, lds + gcol, G, a.tw);
     };
     const cx<T> *in = a.src ? a.src : a.field;

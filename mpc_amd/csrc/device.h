@@ -41,44 +41,32 @@ template <class T> __device__ __forceinline__ void gstore(cx<T> *p, long i, cx<T
 /* ---------------------------------------------------------------------- */
 /* FFT driver: unrolls Plan<N>::R into stages with LDS exchange between    */
 /* ---------------------------------------------------------------------- */
-/*
- * BOFF = 0: one exchange buffer, two barriers per exchange.  BOFF != 0: the
- * stages alternate between lds and lds + BOFF*ls, so a stage's writes can
- * never meet a slower thread's reads of the previous exchange and one
- * barrier per exchange suffices; the caller then puts a barrier before the
- * transform (the buffer it writes first may still be read by the previous
- * user of the LDS).  The sign of BOFF flips at every stage.
- */
-template <class T, int N, int E, int DIR, int PAD, int BOFF, int Ns, int R, int... Rest>
+/* one exchange buffer, two barriers per exchange */
+template <class T, int N, int E, int DIR, int Ns, int R, int... Rest>
 struct DevFft {
     static __device__ __forceinline__ void run(cx<T> (&v)[E], int tid, cx<T> *lds, int ls,
                                                const cx<T> *tw) {
         constexpr bool last = sizeof...(Rest) == 0;
-        fft_stage<T, N, E, R, Ns, DIR, last, PAD>(v, tid, lds, ls, tw);
+        fft_stage<T, N, E, R, Ns, DIR, last, 0>(v, tid, lds, ls, tw);
         if constexpr (!last) {
             __syncthreads();
-            fft_gather<T, N, E, PAD>(v, tid, lds, ls);
-            if constexpr (BOFF == 0) {
-                __syncthreads();
-                DevFft<T, N, E, DIR, PAD, 0, Ns * R, Rest...>::run(v, tid, lds, ls, tw);
-            } else {
-                DevFft<T, N, E, DIR, PAD, -BOFF, Ns * R, Rest...>::run(v, tid, lds + BOFF * ls, ls, tw);
-            }
+            fft_gather<T, N, E, 0>(v, tid, lds, ls);
+            __syncthreads();
+            DevFft<T, N, E, DIR, Ns * R, Rest...>::run(v, tid, lds, ls, tw);
         }
     }
 };
-template <class T, int N, int E, int DIR, int PAD, int BOFF, class Rad> struct DevFftP;
-template <class T, int N, int E, int DIR, int PAD, int BOFF, int... Rs>
-struct DevFftP<T, N, E, DIR, PAD, BOFF, Radices<Rs...>> {
+template <class T, int N, int E, int DIR, class Rad> struct DevFftP;
+template <class T, int N, int E, int DIR, int... Rs>
+struct DevFftP<T, N, E, DIR, Radices<Rs...>> {
     static __device__ __forceinline__ void run(cx<T> (&v)[E], int tid, cx<T> *lds, int ls, const cx<T> *tw) {
-        if constexpr (BOFF != 0) __syncthreads();
-        DevFft<T, N, E, DIR, PAD, BOFF, 1, Rs...>::run(v, tid, lds, ls, tw);
+        DevFft<T, N, E, DIR, 1, Rs...>::run(v, tid, lds, ls, tw);
     }
 };
 /* line FFT with plan PL (PL::E elements per thread, radix list PL::R) */
-template <class T, int N, class PL, int DIR, int PAD = 0, int BOFF = 0>
+template <class T, int N, class PL, int DIR>
 __device__ __forceinline__ void line_fft(cx<T> (&v)[PL::E], int tid, cx<T> *lds, int ls, const cx<T> *tw) {
-    DevFftP<T, N, PL::E, DIR, PAD, BOFF, typename PL::R>::run(v, tid, lds, ls, tw);
+    DevFftP<T, N, PL::E, DIR, typename PL::R>::run(v, tid, lds, ls, tw);
 }
 
 /*
@@ -801,32 +789,27 @@ __device__ __forceinline__ void small_exp(cx<double> x, double &e, double &s, do
 }
 
 /* line FFT with twiddle powers cached per thread (TwChain of the plan) */
-template <class T, int N, int E, int DIR, int PAD, int BOFF, int Ns, int R, int... Rest>
+template <class T, int N, int E, int DIR, int Ns, int R, int... Rest>
 struct DevFftC {
     static __device__ __forceinline__ void run(cx<T> (&v)[E], int tid, cx<T> *lds, int ls,
                                                const TwChain<T, N, E, Ns, R, Rest...> &ch) {
         constexpr bool last = sizeof...(Rest) == 0;
-        fft_stage_t<T, N, E, R, Ns, DIR, last, PAD>(v, tid, lds, ls, TwFromPowers<T, R, E / R, DIR>{ch.p});
+        fft_stage_t<T, N, E, R, Ns, DIR, last, 0>(v, tid, lds, ls, TwFromPowers<T, R, E / R, DIR>{ch.p});
         if constexpr (!last) {
             __syncthreads();
-            fft_gather<T, N, E, PAD>(v, tid, lds, ls);
-            if constexpr (BOFF == 0) {
-                __syncthreads();
-                DevFftC<T, N, E, DIR, PAD, 0, Ns * R, Rest...>::run(v, tid, lds, ls, ch.next);
-            } else {
-                DevFftC<T, N, E, DIR, PAD, -BOFF, Ns * R, Rest...>::run(v, tid, lds + BOFF * ls, ls, ch.next);
-            }
+            fft_gather<T, N, E, 0>(v, tid, lds, ls);
+            __syncthreads();
+            DevFftC<T, N, E, DIR, Ns * R, Rest...>::run(v, tid, lds, ls, ch.next);
         }
     }
 };
 template <class T, int N, int E, class Rad> struct ChainOf;
 template <class T, int N, int E, int... Rs> struct ChainOf<T, N, E, Radices<Rs...>> {
     using type = TwChain<T, N, E, 1, Rs...>;
-    /* line FFT with the thread's cached twiddle powers; BOFF as for DevFft */
-    template <int DIR, int PAD, int BOFF = 0>
+    /* line FFT with the thread's cached twiddle powers */
+    template <int DIR>
     static __device__ __forceinline__ void fft(cx<T> (&v)[E], int tid, cx<T> *lds, int ls, const type &ch) {
-        if constexpr (BOFF != 0) __syncthreads();
-        DevFftC<T, N, E, DIR, PAD, BOFF, 1, Rs...>::run(v, tid, lds, ls, ch);
+        DevFftC<T, N, E, DIR, 1, Rs...>::run(v, tid, lds, ls, ch);
     }
 };
 struct NoChain {};

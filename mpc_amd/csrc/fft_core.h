@@ -354,7 +354,10 @@ MPC_HD void fft_gather(cx<T> (&v)[E], int tid, const cx<T> *lds, int ls) {
 template <int... Rs> struct Radices {};
 
 /* t lines: 8 elements per thread keeps the fused nonlinear kernel's register
- * footprint low (two line copies live at once) */
+ * footprint low (two line copies live at once).  Past 512 points the kernels
+ * take E only (TCross joins 512-point transforms); those radix lists, Plan's
+ * for t lines below and the padded and swizzled maps above are the stage
+ * emulation's, which runs the butterflies, twiddles and exchanges through them */
 template <int N> struct TPlan;
 template <> struct TPlan<4096> { static constexpr int E = 8; using R = Radices<8, 8, 8, 8>; };
 template <> struct TPlan<2048> { static constexpr int E = 8; using R = Radices<8, 8, 8, 4>; };
@@ -454,7 +457,7 @@ template <class T, int NT, int R1, int E> struct TCross {
 };
 
 template <int N> struct Plan;
-/* t lines */
+/* t lines (512: x / y lines too) */
 template <> struct Plan<4096> { static constexpr int E = 16; using R = Radices<16, 16, 16>; };
 template <> struct Plan<2048> { static constexpr int E = 16; using R = Radices<16, 16, 8>; };
 template <> struct Plan<1024> { static constexpr int E = 16; using R = Radices<16, 16, 4>; };
