@@ -142,9 +142,11 @@ template <class G> __device__ __forceinline__ void tline_flush_rho(double rmax, 
  * FP32, 48 in FP64) are worth more as another wave per SIMD, whose work covers
  * the loads: three instead of two in FP32 (256x256x2048 1.10 -> 1.03 ms,
  * 128x128x512 60 -> 56 us), two instead of one in FP64 (2.55 -> 1.88 ms, 137 ->
- * 108 us, 64x64x512 39 -> 31 us; now at least level with the per-group form up
- * to 2048 points).  An FP32 4096-point line's workgroup of eight waves leaves
- * room for two per SIMD only (160 against 175 us at 64x64x4096).
+ * 108 us, 64x64x512 39 -> 31 us; level with the per-group form or faster up to
+ * 2048 points; at 4096 it spills 53 registers and takes 314 us against the
+ * per-group form's 278 at 64x64x4096, 574 before).  An FP32 4096-point line's
+ * workgroup of eight waves leaves room for two per SIMD only (160 against 175 us
+ * at 64x64x4096).
  */
 template <class T, class G, bool PERSIST> constexpr bool TLinePre = PERSIST && sizeof(T) == 4 && G::NT == 4096;
 /* waves per SIMD the kernel is held to */

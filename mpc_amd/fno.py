@@ -11,12 +11,14 @@ channels.  Layers:
     y = Q2 GELU(Q1 v_L + q1) + q2                       (project, W -> H -> 2)
     pred = x[:, :2] + y                                 (the network learns the change over a pass)
 
-Every dense contraction -- the truncated DFTs along t, y and x written as
-real GEMMs against cos/sin matrices, the per-mode complex channel mixing,
-the pointwise channel maps and every transpose of these in the backward
-pass -- runs through mpc_gemm_bf16 (BF16 operands on the matrix cores, FP32
-accumulation).  The backward pass is written out by hand below; there is no
-autograd.  Device buffers come from the library (mpc_dev_*), and every kernel
+The truncated DFTs along t, y and x are real products against cos/sin
+matrices, and they, their transposes in the backward pass and the channel
+maps' weight gradients take BF16 operands on the matrix cores with FP32
+accumulation; the channel maps and the per-mode complex mixing are FP32.
+Networks of the sizes FnoGpu._fits accepts run fused kernels (mpc_fno_column,
+mpc_fno_dft, mpc_fno_wgrad), others the separate ones (mpc_gemm_bf16,
+mpc_fno_combine, mpc_fno_pointwise); both round the same operands in the same
+places.  The backward pass is written out by hand below; there is no autograd.  Device buffers come from the library (mpc_dev_*), and every kernel
 runs on the default stream.
 """
 from __future__ import annotations
@@ -479,8 +481,9 @@ class FnoGpu:
 
     # ---- network ---------------------------------------------------------------
     def _fits(self):
-        """whether the fused kernels take this network's sizes (they hold a whole t-line of every channel in a
-        workgroup); larger ones run the separate kernels"""
+        """whether the fused kernels take this network's sizes: they hold a whole t-line of every channel in a
+        workgroup, and the backward's transposed transforms contract over 2 X and 2 Y, at most 128; larger networks
+        run the separate kernels, forward and backward"""
         c, L = self.cfg, lib()
         # byte offsets within a sample are 32-bit
         return bool(c.cout == 2 and max(c.width, c.hidden) * c.X * c.Y * max(c.T, 2 * c.mt) <= 1 << 29 and L.mpc_fno_column_fits(c.width, c.cin, c.T, 2 * c.mt, c.hidden) and
