@@ -140,7 +140,7 @@ template <class G> __device__ __forceinline__ void tline_flush_rho(double rmax, 
  * Whether a persistent workgroup loads its next line under the current one's
  * transforms (and keeps the Omega grid in registers).  Those registers (24 in
  * FP32, 48 in FP64) are worth more as another wave per SIMD, whose work covers
- * the loads: three instead of two in FP32 (256x256x2048 1.10 -> 1.03 ms,
+ * the loads: three instead of two in FP32 (256x256x2048 1.10 -> 1.01 ms,
  * 128x128x512 60 -> 56 us), two instead of one in FP64 (2.55 -> 1.88 ms, 137 ->
  * 108 us, 64x64x512 39 -> 31 us; level with the per-group form or faster up to
  * 2048 points; at 4096 it spills 53 registers and takes 314 us against the
